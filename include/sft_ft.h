@@ -40,9 +40,12 @@ extern "C" {
 #define SFT_EUNSUPPORTED (-4)
 
 /* sft_ft_fwd_f32_ex flags */
-#define SFT_FWD_AUTO 0x0u /* tiled gather when the shape allows it and the workspace
-                             suffices, otherwise the row gather               */
+#define SFT_FWD_AUTO 0x0u /* tiled gather when the shape allows it, the batch is large
+                             enough for its copy of the table to pay and the
+                             workspace suffices, otherwise the row gather      */
 #define SFT_FWD_ROWS 0x1u /* always the row gather (workspace unused)        */
+#define SFT_FWD_TILES 0x2u /* the tiled gather whatever the batch, when the shape
+                             allows it and the workspace suffices             */
 
 /* sft_ft_bwd_f32 flags */
 #define SFT_BWD_ACCUMULATE 0x0u /* dW[f] += ..., db += ...  (reference semantics)  */

@@ -17,6 +17,7 @@ int fwd_i16(const int32_t *idx, int64_t B, int K, const int16_t *W, int64_t N, i
 int quantize_i16(const float *x, int64_t n, float scale, int16_t *out, hipStream_t s);
 size_t fwd_tiled_workspace(int64_t B, int K, int64_t N, int L);
 bool fwd_tiled_supported(int64_t N, int L, const void *W, const void *bias, const void *out);
+bool fwd_tiled_pays(int64_t B, int K, int64_t N, int L);
 int fwd_f32_tiled(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int L, const float *bias, float *out,
                   void *ws, size_t ws_bytes, hipStream_t s);
 int bwd_workspace(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *bytes);
@@ -268,6 +269,15 @@ bool bad_sizes(int64_t B, int32_t K, int64_t N, int32_t L, std::string &why) {
   return true;
 }
 
+// The forward's flags: at most one of rows and tiles.
+bool bad_fwd_flags(uint32_t flags) {
+  return (flags & ~(SFT_FWD_ROWS | SFT_FWD_TILES)) || flags == (SFT_FWD_ROWS | SFT_FWD_TILES);
+}
+// Whether the flags, or without any the sizes, ask for the tiled gather.
+bool fwd_tiles(int64_t B, int32_t K, int64_t N, int32_t L, uint32_t flags) {
+  return (flags & SFT_FWD_TILES) || (!(flags & SFT_FWD_ROWS) && fwd_tiled_pays(B, K, N, L));
+}
+
 }  // namespace
 
 namespace sft {
@@ -314,8 +324,9 @@ int sft_ft_fwd_f32_workspace_size(int64_t batch, int32_t max_active, int64_t num
   if (!bytes) return fail(SFT_EINVAL, "sft_ft_fwd_f32_workspace_size: null pointer");
   if (bad_sizes(batch, max_active, num_inputs, output_size, why))
     return fail(SFT_EINVAL, "sft_ft_fwd_f32_workspace_size: " + why);
-  if (flags & ~SFT_FWD_ROWS) return fail(SFT_EINVAL, "sft_ft_fwd_f32_workspace_size: unknown flags");
-  const bool tiled = !(flags & SFT_FWD_ROWS) && fwd_tiled_supported(num_inputs, output_size, nullptr, nullptr, nullptr);
+  if (bad_fwd_flags(flags)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_workspace_size: unknown flags");
+  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
+                     fwd_tiled_supported(num_inputs, output_size, nullptr, nullptr, nullptr);
   *bytes = tiled ? fwd_tiled_workspace(batch, max_active, num_inputs, output_size) : 0;
   return SFT_OK;
 }
@@ -327,9 +338,10 @@ int sft_ft_fwd_f32_ex(const int32_t *idx, int64_t batch, int32_t max_active, con
   std::string why;
   if (bad_sizes(batch, max_active, num_inputs, output_size, why)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_ex: " + why);
   if (!weight || !bias || (batch > 0 && (!idx || !out))) return fail(SFT_EINVAL, "sft_ft_fwd_f32_ex: null pointer");
-  if (flags & ~SFT_FWD_ROWS) return fail(SFT_EINVAL, "sft_ft_fwd_f32_ex: unknown flags");
+  if (bad_fwd_flags(flags)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_ex: unknown flags");
   if (batch == 0) return SFT_OK;
-  const bool tiled = !(flags & SFT_FWD_ROWS) && fwd_tiled_supported(num_inputs, output_size, weight, bias, out) &&
+  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
+                     fwd_tiled_supported(num_inputs, output_size, weight, bias, out) &&
                      workspace != nullptr &&
                      workspace_bytes >= fwd_tiled_workspace(batch, max_active, num_inputs, output_size);
   if (tiled)
@@ -370,7 +382,7 @@ int sft_ft_fwd_f32_prep(const int32_t *idx, int64_t batch, int32_t max_active, c
   std::string why;
   if (bad_sizes(batch, max_active, num_inputs, output_size, why)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_prep: " + why);
   if (!weight || !bias || (batch > 0 && (!idx || !out))) return fail(SFT_EINVAL, "sft_ft_fwd_f32_prep: null pointer");
-  if (flags & ~SFT_FWD_ROWS) return fail(SFT_EINVAL, "sft_ft_fwd_f32_prep: unknown flags");
+  if (bad_fwd_flags(flags)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_prep: unknown flags");
   if (bwd_flags & ~(SFT_BWD_OVERWRITE | SFT_BWD_ATOMIC | SFT_BWD_ROWS | SFT_BWD_PREPARED))
     return fail(SFT_EINVAL, "sft_ft_fwd_f32_prep: unknown backward flags");
   if (batch == 0) return SFT_OK;
@@ -391,7 +403,8 @@ int sft_ft_fwd_f32_prep(const int32_t *idx, int64_t batch, int32_t max_active, c
   SideJoinGuard side_join(s);
   if ((rc = bwd_prepare(idx, batch, max_active, num_inputs, output_size, bwd_flags, prep, prep_bytes, side)) != SFT_OK)
     return rc;
-  const bool tiled = !(flags & SFT_FWD_ROWS) && fwd_tiled_supported(num_inputs, output_size, weight, bias, out) &&
+  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
+                     fwd_tiled_supported(num_inputs, output_size, weight, bias, out) &&
                      workspace != nullptr &&
                      workspace_bytes >= fwd_tiled_workspace(batch, max_active, num_inputs, output_size);
   rc = tiled ? fwd_f32_tiled(idx, batch, max_active, weight, num_inputs, output_size, bias, out, workspace,

@@ -49,7 +49,7 @@ template <typename T, int G, int CPL, int U>
 __global__ __launch_bounds__(kBlock) void fwd_f32_kernel(const int32_t *__restrict__ idx, int64_t B, int K, int N,
                                                          const T *__restrict__ W, int64_t cols,
                                                          const T *__restrict__ bias, T *__restrict__ out, int kpad) {
-  static_assert(U == 4, "index reads are 4-wide");
+  static_assert(U % 4 == 0, "index reads are 4-wide");
   constexpr int PPW = kWave / G;
   static_assert(PPW <= kCompactRows, "compact_rows takes at most kCompactRows rows");
   extern __shared__ int smem[];
@@ -79,11 +79,16 @@ __global__ __launch_bounds__(kBlock) void fwd_f32_kernel(const int32_t *__restri
 
   int k = 0;
   for (; k + U <= nmin; k += U) {
-    i32x4 f4 = read4(mylist, k);
+    int fi[U];
+#pragma unroll
+    for (int u = 0; u < U; u += 4) {
+      const i32x4 f4 = read4(mylist, k + u);
+      fi[u] = f4[0], fi[u + 1] = f4[1], fi[u + 2] = f4[2], fi[u + 3] = f4[3];
+    }
     T w[U][CPL];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      int f = f4[u];
+      int f = fi[u];
       if (G == kWave) f = uniform(f);
       const T *row = W + (int64_t)f * cols + c0;
 #pragma unroll
@@ -97,12 +102,17 @@ __global__ __launch_bounds__(kBlock) void fwd_f32_kernel(const int32_t *__restri
         if (colok[j]) acc[j] += w[u][j];
   }
   for (; k < nmax; k += U) {
-    i32x4 f4 = read4(mylist, k);
+    int fi[U];
+#pragma unroll
+    for (int u = 0; u < U; u += 4) {
+      const i32x4 f4 = read4(mylist, k + u);
+      fi[u] = f4[0], fi[u + 1] = f4[1], fi[u + 2] = f4[2], fi[u + 3] = f4[3];
+    }
     T w[U][CPL];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bool v = k + u < n;
-      int f = v ? f4[u] : 0;
+      int f = v ? fi[u] : 0;
       if (G == kWave) f = uniform(f);
       const T *row = W + (int64_t)f * cols + c0;
 #pragma unroll
@@ -1370,19 +1380,37 @@ size_t index_lds_bytes(int G, int K) {
   return (size_t)(kWavesPerBlock * ppw * round_up4(K) + kWavesPerBlock * ppw) * sizeof(int);
 }
 
+// Chunks per lane of the row gather's few-position mapping, 0 for the general one.
+constexpr int64_t kFewWaves = 8192;  // 8 per SIMD: as many as run at once
+static int few_positions_cpl(int64_t B, int64_t cols) {
+  if (B * ceil_div(cols, (int64_t)kWave) <= kFewWaves) return 1;
+  if (B * ceil_div(cols, (int64_t)2 * kWave) <= kFewWaves) return 2;
+  return 0;
+}
+
 int fwd_f32(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int L, const float *bias, float *out,
             hipStream_t s) {
   const bool vec = (L % 4 == 0) && ((uintptr_t)W % 16 == 0) && ((uintptr_t)bias % 16 == 0) &&
                    ((uintptr_t)out % 16 == 0);
   const int64_t cols = vec ? L / 4 : L;
-  const Mapping m = choose_mapping(cols);
+  Mapping m = choose_mapping(cols);
+  // Few positions: a wave per position and 64 or 128 chunks of it, so that the
+  // launch still has waves for every CU and each keeps 16 (8) rows in flight:
+  // a position's rows are one chain of U-row steps, each a memory round trip
+  // (L = 1048: B = 256, K = 32 12.4 -> 5.9 us; B = 64, K = 160 46 -> 14 us).
+  const int few = vec ? few_positions_cpl(B, cols) : 0;
+  if (few > 0) m = Mapping{kWave, few, (int)ceil_div(cols, (int64_t)kWave * few)};
   const int ppb = kWavesPerBlock * (kWave / m.G);
   const dim3 grid((unsigned)ceil_div(B, ppb), (unsigned)m.slabs);
-  const size_t lds = index_lds_bytes(m.G, K);
+  const int kpad = few > 0 ? (K + 15) / 16 * 16 : round_up4(K);  // whole U-row steps of a list
+  const size_t lds = index_lds_bytes(m.G, kpad);
   if (lds > kMaxIndexLds) return fail(SFT_EUNSUPPORTED, "sft_ft_fwd_f32: max_active too large for the LDS index lists");
-  const int kpad = round_up4(K);
   ProfScope prof(kProfFwdF32, s);
-  if (vec) {
+  if (few > 0) {
+    hipLaunchKernelGGL((few == 1 ? fwd_f32_kernel<f32x4, 64, 1, 16> : fwd_f32_kernel<f32x4, 64, 2, 8>), grid,
+                       dim3(kBlock), lds, s, idx, B, K, (int)N, reinterpret_cast<const f32x4 *>(W), cols,
+                       reinterpret_cast<const f32x4 *>(bias), reinterpret_cast<f32x4 *>(out), kpad);
+  } else if (vec) {
     SFT_G_CASES(launch_fwd_f32, f32x4, grid, lds, s, idx, B, K, (int)N, W, cols, bias, out, kpad)
   } else {
     SFT_G_CASES(launch_fwd_f32, float, grid, lds, s, idx, B, K, (int)N, W, cols, bias, out, kpad)
@@ -1527,6 +1555,25 @@ size_t fwd_tiled_workspace(int64_t B, int K, int64_t N, int L) {
 bool fwd_tiled_supported(int64_t N, int L, const void *W, const void *bias, const void *out) {
   return L % 4 == 0 && ceil_div(L, kTileF) >= SFT_FWD_MIN_TILES && N * kTileF * 4 <= (int64_t)(SFT_FWD_TILE_MAX_BYTES) &&
          (uintptr_t)W % 16 == 0 && (uintptr_t)bias % 16 == 0 && (uintptr_t)out % 16 == 0;
+}
+
+// Whether the tiled gather of a shape it supports is the faster one.  It copies
+// the whole table first (2 T bytes at 5 TB/s, then the rank lists: about 6 us,
+// 26 us for lists of more than 32 slots, and 12 us a further table part); the row gather reads only the rows
+// it sums, but from beyond L2, so per byte it loses `slower`: the bytes of rows
+// (three quarters of the slots active) at which the two meet, per us of that
+// first cost, fall as the table outgrows the 4 MB L2s.  Tiled / row gather, us,
+// around the line (N, K, L, B):
+//   23 232, 32, 1048: 3072 55 / 47, 4096 59 / 62;  520: 3072 32 / 28, 4096 34 / 36
+//   8192, 32, 1048: 1536 27 / 23, 2048 29 / 31;  264: 12 288 29 / 27, 16 384 32 / 35
+//   517, 32, 1048: 8192 40 / 39, 16 384 65 / 68
+//   85 296, 160, 1048: 6144 382 / 372, 8192 428 / 488;  136: 12 288 111 / 108
+// and far from it: 23 232, 32, 1048, B = 256 42 / 5.9, B = 65 536 285 / 930.
+bool fwd_tiled_pays(int64_t B, int K, int64_t N, int L) {
+  const double table_mb = 4e-6 * N * L, rows_mb = 3e-6 * B * K * L;
+  const int parts = table_parts(N);
+  const double slower = parts > 1 ? 13 : table_mb > 20 ? 9 : table_mb > 14 ? 12 : table_mb > 4.5 ? 35 : 100;
+  return rows_mb > slower * (0.4 * table_mb + (K <= kRankStageMaxPad ? 6 : 26) + 12 * (parts - 1));
 }
 
 int fwd_f32_tiled(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int L, const float *bias, float *out,

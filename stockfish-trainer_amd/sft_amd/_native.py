@@ -25,6 +25,7 @@ SFT_EWORKSPACE = -2
 SFT_EUNSUPPORTED = -4
 SFT_FWD_AUTO = 0x0
 SFT_FWD_ROWS = 0x1
+SFT_FWD_TILES = 0x2
 SFT_BWD_ACCUMULATE = 0x0
 SFT_BWD_OVERWRITE = 0x1
 SFT_BWD_SORTED = 0x00
@@ -208,12 +209,15 @@ def _on_gpu(device: torch.device, *tensors: torch.Tensor) -> None:
 
 
 def ft_fwd_f32(idx: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out: torch.Tensor,
-               rows: bool = False) -> None:
+               rows: bool = False, tiles: bool = False) -> None:
     """out[b] = bias + sum of weight rows selected by idx[b] (reference order, bit-exact).
 
-    By default the library's tiled gather runs when the shape allows it, with a
-    workspace taken from torch's allocator; rows=True forces the row gather.
+    By default the library's tiled gather runs when the shape allows it and the
+    batch is large enough for it to pay, with a workspace taken from torch's
+    allocator; rows=True forces the row gather, tiles=True the tiled gather
+    where the shape allows it.
     """
+    _require(not (rows and tiles), "rows and tiles exclude each other")
     _require(idx.dim() == 2 and idx.dtype == torch.int32, "idx must be int32 [B, K]")
     _require(weight.dim() == 2 and weight.dtype == torch.float32, "weight must be float32 [N, L]")
     B, K = idx.shape
@@ -221,7 +225,7 @@ def ft_fwd_f32(idx: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out:
     _require(bias.shape == (L,) and bias.dtype == torch.float32, "bias must be float32 [L]")
     _require(out.shape == (B, L) and out.dtype == torch.float32, "out must be float32 [B, L]")
     _on_gpu(idx.device, idx, weight, bias, out)
-    flags = SFT_FWD_ROWS if rows else SFT_FWD_AUTO
+    flags = SFT_FWD_ROWS if rows else SFT_FWD_TILES if tiles else SFT_FWD_AUTO
     nbytes = _workspace_bytes("fwd", B, K, N, L, flags, idx.device)
     ws, ptr = _workspace(nbytes, idx.device)
     with torch.cuda.device(idx.device):

@@ -52,6 +52,27 @@ def test_fwd_matches_oracle(seed, B, N, K, L, lo, hi, sort, rows):
     assert rel_err(y, ft_oracle.fwd_f64(idx, W, b)) <= 1e-5
 
 
+@pytest.mark.parametrize("seed,B,N,K,L,lo,hi,sort", SHAPES)
+def test_fwd_tiles_at_every_batch(seed, B, N, K, L, lo, hi, sort):
+    """The tiled gather at batches for which the library prefers the row gather."""
+    announce(f"fwd tiles seed={seed} B={B} N={N} K={K} L={L}")
+    idx, W, b, _ = case(seed, B, N, K, L, lo, hi, sort)
+    out = torch.empty(B, L, device=DEV)
+    _native.ft_fwd_f32(dev(idx), dev(W), dev(b), out, tiles=True)
+    assert np.array_equal(host(out), ft_oracle.fwd_f32(idx, W, b))
+
+
+# the row gather's mapping by batch: a wave per position and 64 chunks of it (up to 8192 waves), 128 chunks, rows
+@pytest.mark.parametrize("B,N,K,L", [(1, 40, 1, 4), (8192, 300, 3, 256), (8193, 300, 3, 256), (4096, 64, 17, 512),
+                                     (4097, 64, 17, 516), (33, 5000, 160, 1048), (2731, 90, 16, 1500)])
+def test_fwd_rows_few_positions(B, N, K, L):
+    announce(f"fwd rows, few positions B={B} N={N} K={K} L={L}")
+    idx, W, b, _ = case(B, B, N, K, L)
+    out = torch.empty(B, L, device=DEV)
+    _native.ft_fwd_f32(dev(idx), dev(W), dev(b), out, rows=True)
+    assert np.array_equal(host(out), ft_oracle.fwd_f32(idx, W, b))
+
+
 def test_fwd_repeated_feature_and_last_row():
     announce("fwd repeated features, index N-1")
     N, L = 40, 64
