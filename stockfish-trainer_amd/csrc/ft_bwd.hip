@@ -545,6 +545,39 @@ __device__ __forceinline__ void bwd_tile_sum(const P *list, int n, int nmin, int
   }
 }
 
+// bwd_tile_sum for a one-chunk batch of several tiles a workgroup: the sum
+// starts at acc, and without the rolling window, which costs more than it hides
+// over such a batch's shorter lists (B = 8192, two tiles: 110 -> 104 us).
+template <int TCH, typename P>
+__device__ __forceinline__ void bwd_list_sum(const P *list, int n, int nmin, int nmax, int t,
+                                             const char *__restrict__ gtile, f32x4 &acc) {
+  constexpr int U = TCH;
+  const uint32_t lane_off = (uint32_t)t * (uint32_t)sizeof(f32x4);
+  auto row = [&](int b) {
+    return *reinterpret_cast<const f32x4 *>(gtile + ((uint32_t)b * (uint32_t)(TCH * sizeof(f32x4)) + lane_off));
+  };
+  int k = 0;
+  for (; k + U <= nmin; k += U) {
+    f32x4 w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = row((int)list[k + u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc += w[u];
+  }
+  for (; k < nmax; k += U) {
+    f32x4 w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int b = (k + u < n) ? (int)list[k + u] : 0;
+      w[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (k + u < n) w[u] = row(b);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k + u < n) acc += w[u];
+  }
+}
+
 // The 32 features of a workgroup are consecutive, so their position lists
 // form one contiguous range of the sorted array; it is copied to LDS and read
 // from there, which keeps the position reads off the in-order vector-memory
@@ -649,6 +682,7 @@ struct TiledArgs {
   int64_t bcols;
   f32x4 *db;
   int boverwrite;
+  int tile_group;  // tiles per workgroup (1: the single-tile kernel)
 };
 
 // Long-segment slot it.chunk of tile it.tile (whole workgroup).
@@ -663,8 +697,9 @@ __device__ __forceinline__ void tiled_long_item(const TiledArgs &a, TileItem it,
   }
 }
 
-// Feature block it.chunk of tile it.tile (whole workgroup; one barrier inside).
-template <bool NT, bool P16>
+// Feature block it.chunk of tile it.tile, or (MT) of the tile_group tiles from
+// tile_group * it.tile (whole workgroup; one barrier inside).
+template <bool NT, bool P16, bool MT>
 __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem it, char *gsm, int *s_seg,
                                                    int *s_perm) {
   constexpr int TCH = kBwdTileCh;
@@ -734,7 +769,7 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
       }
     }
   }
-  if (lay.plus >= 0) {
+  if (!MT && lay.plus >= 0) {
     const int colm = tile_col(map, it.tile, cs);
     f32x4 vp = f32x4{0.f, 0.f, 0.f, 0.f};
     if (fs < N && colm >= 0 && !long_segment(as, es)) {
@@ -769,6 +804,26 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
   const int n = (live && !is_long) ? s1 - s0 : 0;
   int nmin, nmax;
   group_minmax<TCH>(n, nmin, nmax);
+  if (MT) {
+    // one position chunk: the sums start at 0, and the dW_0 rows of kDstOutPlus
+    // are loaded by the lane that adds onto them, with its first row loads
+    const int t0 = it.tile * a.tile_group, t1 = min(t0 + a.tile_group, a.ntiles);
+    const int blk = block_of(live ? f : fb, dst.n, dst.start);
+    f32x4 *drow = pick(dst.p, blk) + ((live ? f : fb) - pick(dst.start, blk)) * cols4;
+    for (int tile = t0; tile < t1; ++tile) {  // workgroup-uniform
+      const int colm = tile_col(map, tile, t);
+      const bool store = live && !is_long && colm >= 0;
+      const char *gtile = reinterpret_cast<const char *>(gt + (int64_t)tile * B * TCH);
+      f32x4 plus = f32x4{0.f, 0.f, 0.f, 0.f}, acc = plus;
+      if (dst_mode == kDstOutPlus && store) plus = load_row<NT>(drow + colm);
+      if (staged)
+        bwd_list_sum<TCH>(spos + (s0 - ra), n, nmin, nmax, t, gtile, acc);
+      else
+        bwd_list_sum<TCH>(sorted_pos + s0, n, nmin, nmax, t, gtile, acc);
+      if (store) store_row<NT>(drow + colm, dst_mode == kDstOutPlus ? plus + acc : acc);
+    }
+    return;
+  }
   const int colm = tile_col(map, it.tile, t);
   const bool colok = colm >= 0;
   const char *gtile = reinterpret_cast<const char *>(gt + (int64_t)it.tile * B * TCH);
@@ -801,7 +856,7 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
 // long-segment slots first, then the feature blocks); workgroups after the
 // items, when the launch carries them, reduce the bias partials (the bias
 // pass's second step, which then needs no launch of its own).
-template <bool NT, bool P16>
+template <bool NT, bool P16, bool MT>
 __global__ __launch_bounds__(kBlock) void bwd_tiled_gather_kernel(TiledArgs a) {
   extern __shared__ __align__(16) char gsm[];
   __shared__ int s_seg[kBwdFeat + 1], s_perm[kBwdFeat];
@@ -811,15 +866,53 @@ __global__ __launch_bounds__(kBlock) void bwd_tiled_gather_kernel(TiledArgs a) {
   }
   const int64_t nl_items = tile_sched_items_per_xcd(a.ntiles, a.nlong) * kXcds;
   const bool long_item = (int64_t)blockIdx.x < nl_items;  // whole block: uniform
-  const TileItem it = long_item ? tile_sched_item(blockIdx.x, a.ntiles, a.nlong)
-                                : tile_sched_item(blockIdx.x - nl_items, a.ntiles, a.ngroups);
-  if (it.tile >= a.ntiles) return;  // whole block: uniform
+  const int nt = MT && !long_item ? (a.ntiles + a.tile_group - 1) / a.tile_group : a.ntiles;
+  const TileItem it = long_item ? tile_sched_item(blockIdx.x, nt, a.nlong)
+                                : tile_sched_item(blockIdx.x - nl_items, nt, a.ngroups);
+  if (it.tile >= nt) return;  // whole block: uniform
   if (long_item)
     tiled_long_item(a, it, gsm);
   else
-    tiled_feature_item<NT, P16>(a, it, gsm, s_seg, s_perm);
+    tiled_feature_item<NT, P16, MT>(a, it, gsm, s_seg, s_perm);
 }
 
+
+// A batch whose whole grad tile fits an XCD's L2 (4 MB: B <= 32768) is gathered
+// in one position chunk: no partial weight grads to store and reload (B = 16384:
+// 0.768 -> 0.619 ms per step, B = 32768: 1.139 -> 0.998 ms).  At B = 65536 one
+// chunk of 8.4 MB thrashes the L2 (1.84 -> 2.03 ms).
+#ifndef SFT_BWD_ONE_CHUNK_BYTES
+#define SFT_BWD_ONE_CHUNK_BYTES (4 << 20)
+#endif
+// Whether a one-chunk batch's weight grad is gathered by rows: with few slots
+// per feature the tiled launch is mostly workgroups with little to sum, and the
+// row gather (one wave a feature, its whole row at once) needs no grad tiles.
+// Backward, tiled (several tiles a workgroup, below) / rows, us (N, K, L, B):
+// 23 232, 32, 1048: 256 84 / 56, 2904 92 / 86, 4356 97 / 105;  520: 2904 72 / 63,
+// 5808 78 / 81;  85 296, 160, 1048: 2132 204 / 173, 3198 224 / 226;  4096, 32,
+// 1048: 512 55 / 47, 1536 59 / 58;  517: even.
+bool few_slots(int64_t B, int K, int64_t N) {
+  return B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) && B * (int64_t)K <= 4 * N;
+}
+
+// Tiles per workgroup of a one-chunk gather.  A feature block's segment bounds,
+// positions and ranking are the same for every column tile, and with few
+// positions they are most of a workgroup's time (three dependent round trips
+// before its first row), so a workgroup takes two tiles with one such prologue
+// when both tiles' grad rows fit an XCD's L2 (B <= 16 384) and the launch keeps
+// two rounds of resident workgroups (256 CUs x 7): narrow rows and small tables
+// keep one.  Backward with 1 / 2 / 4 tiles, us: N = 23 232, L = 1048, uniform
+// rows, B = 3500 112 / 94 / 85, B = 8192 123 / 104 / 104, B = 16 384 147 / 139
+// / 179, B = 32 768 233 / 316 / 414; encoded positions (a workgroup lasts as
+// long as its longest list times its tiles), B = 5003 139 / 135 / 157, B = 16 384
+// 151 / 133 / 132; L = 136, B = 8192 57 / 57 / 60; N = 2048, B = 8192 95 / 99 / 105.
+constexpr int kGatherTileGroup = 2;
+constexpr int64_t kGatherMinBlocks = 2 * 256 * 7;
+int gather_tile_group(int64_t B, int ntiles, int64_t ngroups) {
+  const int64_t l2 = ((int64_t)4 << 20) / (std::max<int64_t>(B, 1) * 16 * kBwdTileCh);
+  const int64_t fill = ngroups * ntiles / kGatherMinBlocks;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({l2, fill, (int64_t)kGatherTileGroup}));
+}
 
 // One position chunk's tiled weight-grad gather.
 // pos16: the slots' 16-bit chunk offsets (null when a chunk has more than
@@ -837,19 +930,26 @@ int launch_tiled_gather(bool nt, const int32_t *seg, const int32_t *pos, const u
                         int64_t N, const f32x4 *gt, int64_t B, const ColMap &map, const RowDst &dst, f32x4 *tmp,
                         int src_mode, int dst_mode, int ntiles, int ngroups, const int32_t *long_list,
                         const int *long_count, int nlong, hipStream_t s, const BiasFinal *bias = nullptr) {
-  const int64_t items = tile_sched_items_per_xcd(ntiles, nlong) + tile_sched_items_per_xcd(ntiles, ngroups);
-  const size_t lds = (size_t)gather_lds(dst_mode).bytes;
+  const bool one_chunk = src_mode == kSrcZero && dst_mode != kDstTmp;
+  const int tg = one_chunk && pos16 != nullptr ? gather_tile_group(B, ntiles, ngroups) : 1;
+  const int64_t items = tile_sched_items_per_xcd(ntiles, nlong) +
+                        tile_sched_items_per_xcd((int)ceil_div(ntiles, tg), ngroups);
+  const size_t lds = (size_t)gather_lds(tg > 1 ? kDstOut : dst_mode).bytes;
   if ((uintptr_t)pos % 16 != 0 || (uintptr_t)pos16 % 16 != 0)  // 256-byte / 16-byte aligned workspace regions
     return fail(SFT_EINVAL, "tiled feature gather: sorted positions not 16-byte aligned");
   const int64_t gblocks = items * kXcds;
   const TiledArgs a{seg, pos, pos16, (int)chunk_base, N, gt, B, map, dst, tmp, src_mode, dst_mode, ntiles, ngroups,
                     long_list, long_count, nlong, gblocks, bias ? bias->partial : nullptr, bias ? bias->nparts : 0,
-                    bias ? bias->cols : 0, bias ? bias->db : nullptr, bias ? bias->overwrite : 0};
+                    bias ? bias->cols : 0, bias ? bias->db : nullptr, bias ? bias->overwrite : 0, tg};
   const bool p16 = pos16 != nullptr;
   const dim3 grid((unsigned)(gblocks + (bias ? bias_final_blocks(bias->cols) : 0)));
-  hipLaunchKernelGGL((nt ? (p16 ? bwd_tiled_gather_kernel<true, true> : bwd_tiled_gather_kernel<true, false>)
-                         : (p16 ? bwd_tiled_gather_kernel<false, true> : bwd_tiled_gather_kernel<false, false>)),
-                     grid, dim3(kBlock), lds, s, a);
+  if (tg > 1)
+    hipLaunchKernelGGL((nt ? bwd_tiled_gather_kernel<true, true, true> : bwd_tiled_gather_kernel<false, true, true>),
+                       grid, dim3(kBlock), lds, s, a);
+  else
+    hipLaunchKernelGGL((nt ? (p16 ? bwd_tiled_gather_kernel<true, true, false> : bwd_tiled_gather_kernel<true, false, false>)
+                           : (p16 ? bwd_tiled_gather_kernel<false, true, false> : bwd_tiled_gather_kernel<false, false, false>)),
+                       grid, dim3(kBlock), lds, s, a);
   return check_launch("tiled feature gather");
 }
 
@@ -1169,13 +1269,6 @@ bool tiled_shape(int64_t B, int L, uint32_t flags) {
 #define SFT_BWD_CHUNKS 2
 #endif
 constexpr int kBwdHalves = SFT_BWD_CHUNKS;
-// A batch whose whole grad tile fits an XCD's L2 (4 MB: B <= 32768) is gathered
-// in one position chunk: no partial weight grads to store and reload (B = 16384:
-// 0.768 -> 0.619 ms per step, B = 32768: 1.139 -> 0.998 ms).  At B = 65536 one
-// chunk of 8.4 MB thrashes the L2 (1.84 -> 2.03 ms).
-#ifndef SFT_BWD_ONE_CHUNK_BYTES
-#define SFT_BWD_ONE_CHUNK_BYTES (4 << 20)
-#endif
 int sort_chunks(int64_t B, int L, uint32_t flags) {
   if (!tiled_shape(B, L, flags) || B < kBwdHalves) return 1;
   return B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) ? 1 : kBwdHalves;
@@ -1407,7 +1500,8 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
   // The tiled weight-grad gather reads the grad in column tiles; the bias pass
   // writes that layout while it streams the grad (16-byte loads when the grad
   // allows them, 4-byte loads otherwise), and stores 16-byte weight-grad chunks.
-  const bool tiled = !(flags & SFT_BWD_ATOMIC) && M > 0 && tiled_shape(B, L, flags) && (uintptr_t)dW % 16 == 0;
+  const bool tiled = !(flags & SFT_BWD_ATOMIC) && M > 0 && tiled_shape(B, L, flags) && !few_slots(B, K, N) &&
+                     (uintptr_t)dW % 16 == 0;
   f32x4 *gt = tiled ? reinterpret_cast<f32x4 *>(w + lay.gt) : nullptr;
 
   // ---- sort of the slots and their segments: they need only the indices, so
@@ -1565,7 +1659,8 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
     const int64_t cols = vec ? L / 4 : L;
     const Mapping m = choose_mapping(cols);
     const int fpb = kWavesPerBlock * (kWave / m.G);
-    const int nlong = vec ? kRowLongBlocks : 0;
+    // long segments hold more than kLongSeg slots each: at most M / kLongSeg of them
+    const int nlong = vec ? (int)std::min<int64_t>(kRowLongBlocks, M / kLongSeg * ceil_div(cols, (int64_t)8)) : 0;
     const dim3 grid((unsigned)(nlong + ceil_div(N, fpb)), (unsigned)m.slabs);
     ProfScope prof(kProfBwdGather, s);
     if (vec) {

@@ -95,6 +95,23 @@ def test_sorted_bwd_skewed_segments(seed, B, N, K, L, hot, p_hot, overwrite, row
     assert np.array_equal(dW, rW)
 
 
+# one position chunk, two tiles a workgroup (the last group one tile, or both) and, with at most
+# four slots a feature, the row gather
+@pytest.mark.parametrize("B,N,K,L,hot", [(3001, 23232, 32, 1048, 0), (9000, 14000, 8, 1000, 9), (16384, 8000, 16, 1040, 9),
+                                         (2904, 23232, 32, 1044, 0), (2905, 23232, 32, 1044, 0), (700, 800, 4, 136, 3)])
+def test_sorted_bwd_tile_groups(B, N, K, L, hot):
+    announce(f"bwd tile groups B={B} N={N} K={K} L={L}")
+    g = np.random.default_rng(B)
+    idx = workloads.make_indices(g, B, N, K, 0, K, sort=False)
+    for f in range(hot):  # long segments
+        idx[g.random(B) < 0.3, f % K] = f
+    G = g.standard_normal((B, L)).astype(np.float32)
+    dW, db = run_bwd(idx, G, N, _native.SFT_BWD_OVERWRITE)
+    rW, _ = ft_oracle.bwd_f32(idx, G, N)
+    assert np.array_equal(dW, rW)
+    assert rel_err(db, G.astype(np.float64).sum(0)) <= 1e-5
+
+
 @pytest.mark.parametrize("N", [2500, 1500])
 def test_sorted_bwd_every_segment_long(N):
     """Every feature long (~450 and ~750 slots per position chunk): thousands
