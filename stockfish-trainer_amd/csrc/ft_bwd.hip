@@ -41,10 +41,11 @@ int *slot_sort_positions(int64_t M, int64_t N, int nchunks, void *ws);
 bool slot_sort_buckets_supported(int64_t N, int nchunks);
 int slot_sort_buckets(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, int nchunks, void *ws,
                       int32_t *seg, int32_t *list, int *count, uint16_t *pos16, int long_period, int **pos_sorted,
-                      hipStream_t s);
+                      hipStream_t s, const int32_t *idx1 = nullptr);
+// (idx1: the slots from M / 2 on, a second matrix.)
 // Its two halves: the radix pass into ws, then the buckets from ws (only read).
 int slot_sort_buckets_high(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, int nchunks, void *ws,
-                           int *clear, int nclear, hipStream_t s);
+                           int *clear, int nclear, hipStream_t s, const int32_t *idx1 = nullptr);
 int slot_sort_buckets_low(const void *ws, int64_t M, int64_t N, int chunk_rows, int nchunks, int *vout,
                           int32_t *seg, int32_t *list, int *count, uint16_t *pos16, int long_period, hipStream_t s,
                           int bfirst = 0, int bend = -1);
@@ -72,16 +73,28 @@ constexpr int kBiasMaxParts = SFT_BIAS_PARTS;
 // (long_segment_sum_wg: reserved workgroups of the same gather launch) and
 // skipped by the per-feature lane groups.  Whether segment [s0, s1) of the
 // sorted slots is long depends on its bounds alone, so both sides agree: it
-// is long when it contains two consecutive multiples of kLongSeg ("samples")
-// of the sorted slot index.  Every segment of 2 kLongSeg slots or more is
-// long, none of kLongSeg slots or fewer.  seg_offsets_kernel lists them (per
+// is long when it contains two consecutive multiples of its period ("samples")
+// of the sorted slot index.  Every segment of 2 periods of slots or more is
+// long, none of one period or fewer.  seg_offsets_kernel lists them (per
 // position chunk) as it finds them at their first sample m:
-// keys[m + kLongSeg] == keys[m] != keys[m - kLongSeg].
+// keys[m + period] == keys[m] != keys[m - period].  The period is kLongSeg,
+// shorter for small batches (long_period).
 #ifndef SFT_BWD_LONG_SEG
 #define SFT_BWD_LONG_SEG 128
 #endif
 constexpr int kLongSeg = SFT_BWD_LONG_SEG;
-__host__ __device__ inline bool long_segment(int64_t s0, int64_t s1) { return sft::long_segment(s0, s1, kLongSeg); }
+// A one-chunk batch with few slots a feature takes shorter segments as long:
+// there a feature of 100 positions (each king square's, over encoded positions)
+// keeps its workgroup for many times the others' time, and few features are
+// that long.  Backward of 5003 encoded positions (N = 24 576, K = 32) at 128 / 32,
+// us: L = 1048 136 / 104, both perspectives of the composed table 235 / 166;
+// 16 384 positions (21 slots a feature) 133 / 166, so only up to 12.
+constexpr int kLongSegFew = 32;
+inline int long_period(int64_t B, int K, int64_t N) { return B <= 32768 && B * K <= 12 * N ? kLongSegFew : kLongSeg; }
+static_assert((kLongSeg & (kLongSeg - 1)) == 0, "periods are powers of two");
+__device__ __forceinline__ bool long_segment(int s0, int s1, int period) {  // sft::long_segment, without the division
+  return ((s0 + period - 1) & -period) + period < s1;
+}
 
 // Segment starts and the lists of long segments of one sort: seg[0 .. nc N]
 // (nc position chunks of nfeat features), then per chunk c a list of its long
@@ -116,7 +129,8 @@ __global__ __launch_bounds__(kBlock) void seg_offsets_kernel(const unsigned *__r
                                                              int32_t *__restrict__ long_list,
                                                              int *__restrict__ long_count,
                                                              const int32_t *__restrict__ pos,
-                                                             uint16_t *__restrict__ pos16, int chunk_rows) {
+                                                             uint16_t *__restrict__ pos16, int chunk_rows,
+                                                             int period) {
   __shared__ unsigned s_active;
   if (threadIdx.x < kWave) {
     unsigned v = 0;
@@ -133,7 +147,7 @@ __global__ __launch_bounds__(kBlock) void seg_offsets_kernel(const unsigned *__r
     if (pos16 != nullptr && i < M) pos16[i] = (uint16_t)(pos[i] - (int)(cur / nfeat) * chunk_rows);
     const int64_t hi = cur < N ? cur : N;
     for (int64_t f = prev + 1; f <= hi; ++f) seg_start[f] = (int32_t)i;
-    if (long_listed_at(keys, M, i, kLongSeg)) {
+    if (long_listed_at(keys, M, i, period)) {
       const int64_t c = cur / nfeat;
       const int at = atomicAdd(long_count + c, 1);
       long_list[c * nfeat + at] = (int32_t)(cur - c * nfeat);
@@ -222,15 +236,12 @@ __device__ __forceinline__ void long_store(const LongEnds &e, int dst_mode, floa
 // gather's own sequence, so a feature's result does not depend on the path.
 // Threads kBlock and above of a larger workgroup take part in the barriers only.
 constexpr int kWgLongRows = 128;  // 128 x 128 B = 16 KB of LDS
-__device__ __forceinline__ void long_segment_sum_wg(const int32_t *__restrict__ sorted_pos, int64_t f, int s0, int n,
-                                                    int cb, const LongRows &rows, const ColMap &map,
-                                                    const RowDst &dst, f32x4 *__restrict__ tmp, int64_t nfeat,
-                                                    int src_mode, int dst_mode, f32x4 *buf) {
+__device__ __forceinline__ float long_rows_sum_wg(const int32_t *__restrict__ sorted_pos, int s0, int n, int cb,
+                                                  const LongRows &rows, const ColMap &map, bool col, float acc,
+                                                  f32x4 *buf) {
   constexpr int kRowsPerPass = kBlock / 8;
   constexpr int kPass = kWgLongRows / kRowsPerPass;
   const bool stager = threadIdx.x < kBlock;
-  const LongEnds ends = long_ends(f, cb, (int)threadIdx.x, map, dst, tmp, nfeat);
-  float acc = long_start(ends, src_mode);
   const int q = threadIdx.x & 7, r0 = threadIdx.x >> 3;  // staging: chunk q of rows r0 + 32 u
   const bool qok = tile_col(map, cb, q) >= 0;
   const f32x4 *src = rows.base + cb * rows.blk_stride + q;
@@ -265,7 +276,7 @@ __device__ __forceinline__ void long_segment_sum_wg(const int32_t *__restrict__ 
       load_rows();
       if (b + 2 < nb) load_pos(b + 2);
     }
-    if (ends.ccol >= 0) {
+    if (col) {
       const float *row = reinterpret_cast<const float *>(buf) + threadIdx.x;
       const int nrows = min(kWgLongRows, n - b * kWgLongRows);
 #pragma unroll 16
@@ -275,7 +286,15 @@ __device__ __forceinline__ void long_segment_sum_wg(const int32_t *__restrict__ 
     if (more) stage();
     __syncthreads();
   }
-  long_store(ends, dst_mode, acc);
+  return acc;
+}
+__device__ __forceinline__ void long_segment_sum_wg(const int32_t *__restrict__ sorted_pos, int64_t f, int s0, int n,
+                                                    int cb, const LongRows &rows, const ColMap &map,
+                                                    const RowDst &dst, f32x4 *__restrict__ tmp, int64_t nfeat,
+                                                    int src_mode, int dst_mode, f32x4 *buf) {
+  const LongEnds ends = long_ends(f, cb, (int)threadIdx.x, map, dst, tmp, nfeat);
+  const float start = long_start(ends, src_mode);
+  long_store(ends, dst_mode, long_rows_sum_wg(sorted_pos, s0, n, cb, rows, map, ends.ccol >= 0, start, buf));
 }
 
 // Row gather: the first nlong workgroups (column slab 0) sum the listed long
@@ -287,7 +306,8 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(const int32_t *__re
                                                              const T *__restrict__ grad, int64_t cols,
                                                              T *__restrict__ dW, int overwrite,
                                                              const int32_t *__restrict__ long_list,
-                                                             const int *__restrict__ long_count, int nlong) {
+                                                             const int *__restrict__ long_count, int nlong,
+                                                             int period) {
   if ((int)blockIdx.x < nlong) {  // whole block: uniform
     if constexpr (std::is_same<T, f32x4>::value) {
       __shared__ f32x4 lbuf[kWgLongRows * 8];
@@ -324,7 +344,7 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(const int32_t *__re
     s0 = uniform(s0);
     s1 = uniform(s1);
   }
-  const bool is_long = skip_long && live && long_segment(s0, s1);  // summed by the long-segment blocks
+  const bool is_long = skip_long && live && long_segment(s0, s1, period);  // summed by the long-segment blocks
   const int n = is_long ? 0 : s1 - s0;
   int nmin, nmax;
   group_minmax<G>(n, nmin, nmax);
@@ -683,6 +703,8 @@ struct TiledArgs {
   f32x4 *db;
   int boverwrite;
   int tile_group;  // tiles per workgroup (1: the single-tile kernel)
+  const f32x4 *gt1;  // bwd_pair_gather_kernel: perspective 1's grad tiles
+  int long_period;
 };
 
 // Long-segment slot it.chunk of tile it.tile (whole workgroup).
@@ -695,6 +717,48 @@ __device__ __forceinline__ void tiled_long_item(const TiledArgs &a, TileItem it,
     long_segment_sum_wg(a.sorted_pos, f, s0, a.seg[f + 1] - s0, it.tile, LongRows{a.gt, a.B * TCH, TCH}, a.map,
                         a.dst, a.tmp, a.N, a.src_mode, a.dst_mode, reinterpret_cast<f32x4 *>(gsm));
   }
+}
+
+// Copies cnt4 16-byte pieces of a position stream to LDS, 16-bit offsets (P16)
+// widened to ints, four loads per thread in flight.
+template <bool P16>
+__device__ __forceinline__ void stage_positions(const void *__restrict__ from, int cnt4, int *to) {
+  constexpr int U = 4;
+  const int tid = threadIdx.x;
+  const i32x4 *src = reinterpret_cast<const i32x4 *>(from);
+  i32x4 *dst4 = reinterpret_cast<i32x4 *>(to);
+  for (int b0 = 0; b0 < cnt4; b0 += U * kBlock) {
+    i32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = b0 + u * kBlock + tid;
+      v[u] = i < cnt4 ? SFT_STREAM_LOAD(src + i) : i32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = b0 + u * kBlock + tid;
+      if (i >= cnt4) continue;
+      if (P16) {
+        const uint32_t w0 = (uint32_t)v[u][0], w1 = (uint32_t)v[u][1], w2 = (uint32_t)v[u][2], w3 = (uint32_t)v[u][3];
+        dst4[2 * i] = i32x4{(int)(w0 & 0xffffu), (int)(w0 >> 16), (int)(w1 & 0xffffu), (int)(w1 >> 16)};
+        dst4[2 * i + 1] = i32x4{(int)(w2 & 0xffffu), (int)(w2 >> 16), (int)(w3 & 0xffffu), (int)(w3 >> 16)};
+      } else {
+        dst4[i] = v[u];
+      }
+    }
+  }
+}
+
+// A wave runs as long as its longest segment: wave 0 ranks the block's features
+// (lane l's length is len) by length, ties by index, into s_perm, so that each
+// wave gets 8 consecutive ranks.
+__device__ __forceinline__ void rank_features(int len, int lane, int *s_perm) {
+  int rank = 0;
+  for (int j = 0; j < kBwdFeat; ++j) {
+    const int o = __builtin_amdgcn_readlane(len, j);
+    rank += (o > len || (o == len && j < lane)) ? 1 : 0;
+  }
+  if (lane < kBwdFeat) s_perm[rank] = lane;
 }
 
 // Feature block it.chunk of tile it.tile, or (MT) of the tile_group tiles from
@@ -743,54 +807,22 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
   const int ra = r0 & ~(PER - 1);
   const int cnt4 = (r1 - ra + PER - 1) / PER;           // 16-byte pieces
   const bool staged = cnt4 * PER <= kBwdPosLds;         // block-uniform
-  if (staged) {
-    constexpr int U = 4;
-    const i32x4 *src = P16 ? reinterpret_cast<const i32x4 *>(pos16 + ra)
-                           : reinterpret_cast<const i32x4 *>(sorted_pos + ra);
-    i32x4 *dst4 = reinterpret_cast<i32x4 *>(spos);
-    for (int b0 = 0; b0 < cnt4; b0 += U * kBlock) {
-      i32x4 v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = b0 + u * kBlock + tid;
-        v[u] = i < cnt4 ? SFT_STREAM_LOAD(src + i) : i32x4{0, 0, 0, 0};
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = b0 + u * kBlock + tid;
-        if (i >= cnt4) continue;
-        if (P16) {
-          const uint32_t w0 = (uint32_t)v[u][0], w1 = (uint32_t)v[u][1], w2 = (uint32_t)v[u][2], w3 = (uint32_t)v[u][3];
-          dst4[2 * i] = i32x4{(int)(w0 & 0xffffu), (int)(w0 >> 16), (int)(w1 & 0xffffu), (int)(w1 >> 16)};
-          dst4[2 * i + 1] = i32x4{(int)(w2 & 0xffffu), (int)(w2 >> 16), (int)(w3 & 0xffffu), (int)(w3 >> 16)};
-        } else {
-          dst4[i] = v[u];
-        }
-      }
-    }
-  }
+  if (staged)
+    stage_positions<P16>(P16 ? static_cast<const void *>(pos16 + ra) : static_cast<const void *>(sorted_pos + ra), cnt4,
+                         spos);
   if (!MT && lay.plus >= 0) {
     const int colm = tile_col(map, it.tile, cs);
     f32x4 vp = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (fs < N && colm >= 0 && !long_segment(as, es)) {
+    if (fs < N && colm >= 0 && !long_segment(as, es, a.long_period)) {
       const int blk = block_of(fs, dst.n, dst.start);
       vp = load_row<NT>(pick(dst.p, blk) + (fs - pick(dst.start, blk)) * cols4 + colm);
     }
     reinterpret_cast<f32x4 *>(gsm + lay.plus)[tid] = vp;
   }
   if (wave == 0) {
-    // A wave runs as long as its longest segment: rank the features by segment
-    // length (ties by index, long segments as 0) and give each wave 8
-    // consecutive ranks.
     const int le = __shfl_down(la, 1);
     const bool live = lane < nf;
-    const int len = (live && !long_segment(la, le)) ? le - la : 0;
-    int rank = 0;
-    for (int j = 0; j < kBwdFeat; ++j) {
-      const int o = __builtin_amdgcn_readlane(len, j);
-      rank += (o > len || (o == len && j < lane)) ? 1 : 0;
-    }
-    if (lane < kBwdFeat) s_perm[rank] = lane;
+    rank_features((live && !long_segment(la, le, a.long_period)) ? le - la : 0, lane, s_perm);  // long segments as 0
     if (lane <= kBwdFeat) s_seg[lane] = la;
   }
   __syncthreads();
@@ -800,7 +832,7 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
   const int64_t f = fb + p;
   const int s0 = s_seg[p], s1 = s_seg[p + 1];
   const bool live = p < nf;
-  const bool is_long = live && long_segment(s0, s1);  // summed by the long-segment slots
+  const bool is_long = live && long_segment(s0, s1, a.long_period);  // summed by the long-segment slots
   const int n = (live && !is_long) ? s1 - s0 : 0;
   int nmin, nmax;
   group_minmax<TCH>(n, nmin, nmax);
@@ -877,6 +909,112 @@ __global__ __launch_bounds__(kBlock) void bwd_tiled_gather_kernel(TiledArgs a) {
 }
 
 
+// Both perspectives of a composed table in one launch, for one-chunk batches:
+// dW = dW_0 + dW_1, each summed from 0 over its perspective's positions
+// ascending (two sums and one add, as autograd forms it).  One sort holds both
+// (key = perspective N + feature), so feature f's lists are segments f and N + f,
+// and gt / gt1 hold the perspectives' grad tiles.  As tiled_feature_item<MT>:
+// tile_group tiles share the prologue.  Against two launches, the second adding
+// onto the first's rows, it reads and writes the weight grad once less and
+// starts half the workgroups.  Backward of the composed HalfKAv2_hm table
+// (L = 1048), two launches / one, us: 1000 encoded positions 248 / 142, 5003 315 /
+// 166, 16 384 377 / 287; Full_Threats+HalfKAv2_hm, 5003 830 / 362.
+template <bool NT>
+__global__ __launch_bounds__(kBlock) void bwd_pair_gather_kernel(TiledArgs a) {
+  constexpr int TCH = kBwdTileCh;
+  extern __shared__ __align__(16) char gsm[];
+  __shared__ int s_seg[2][kBwdFeat + 1], s_perm[kBwdFeat];
+  if ((int64_t)blockIdx.x >= a.gblocks) {  // whole block: uniform
+    bias_final_block<f32x4>((int64_t)blockIdx.x - a.gblocks, a.bpart, a.bparts, a.bcols, a.db, a.boverwrite);
+    return;
+  }
+  const int64_t N = a.N;
+  const int64_t nl_items = tile_sched_items_per_xcd(a.ntiles, a.nlong) * kXcds;
+  if ((int64_t)blockIdx.x < nl_items) {  // a long-segment slot: features long in either perspective
+    const TileItem it = tile_sched_item(blockIdx.x, a.ntiles, a.nlong);
+    if (it.tile >= a.ntiles) return;
+    const int c0 = a.long_count[0], cnt = c0 + a.long_count[1];
+    f32x4 *buf = reinterpret_cast<f32x4 *>(gsm);
+    for (int e = it.chunk; e < cnt; e += a.nlong) {  // workgroup-uniform
+      const int64_t f = e < c0 ? a.long_list[e] : a.long_list[N + e - c0];
+      const int s0 = a.seg[f], s1 = a.seg[f + 1], u0 = a.seg[N + f], u1 = a.seg[N + f + 1];
+      if (e >= c0 && long_segment(s0, s1, a.long_period)) continue;  // listed by perspective 0
+      const LongEnds ends = long_ends(f, it.tile, (int)threadIdx.x, a.map, a.dst, nullptr, N);
+      const bool col = ends.ccol >= 0;
+      const float d0 = long_rows_sum_wg(a.sorted_pos, s0, s1 - s0, it.tile, LongRows{a.gt, a.B * TCH, TCH}, a.map, col,
+                                        0.f, buf);
+      // perspective 1's sorted positions follow perspective 0's: B .. 2 B - 1
+      const float d1 = long_rows_sum_wg(a.sorted_pos, u0, u1 - u0, it.tile,
+                                        LongRows{a.gt1 - a.B * TCH, a.B * TCH, TCH}, a.map, col, 0.f, buf);
+      if (col) *ends.dp = d0 + d1;
+    }
+    return;
+  }
+  const int ngrp = (a.ntiles + a.tile_group - 1) / a.tile_group;
+  const TileItem it = tile_sched_item(blockIdx.x - nl_items, ngrp, a.ngroups);
+  if (it.tile >= ngrp) return;  // whole block: uniform
+  const int tid = threadIdx.x, wave = uniform(tid / kWave), lane = tid % kWave;
+  const int64_t fb = (int64_t)it.chunk * kBwdFeat;
+  const int nf = (int)(N - fb < kBwdFeat ? N - fb : kBwdFeat);
+  int *spos = reinterpret_cast<int *>(gsm);
+  // as in tiled_feature_item: the ranges' bounds, then their positions
+  int r0[2], r1[2], la[2] = {0, 0};
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    r0[p] = a.seg[p * N + fb];
+    r1[p] = a.seg[p * N + fb + nf];
+    if (wave == 0) la[p] = a.seg[p * N + fb + (lane < nf ? lane : nf)];
+  }
+  constexpr int PER = 8;
+  const int ra0 = r0[0] & ~(PER - 1), ra1 = r0[1] & ~(PER - 1);
+  const int cnt0 = (r1[0] - ra0 + PER - 1) / PER, cnt1 = (r1[1] - ra1 + PER - 1) / PER;
+  const bool staged = (cnt0 + cnt1) * PER <= kBwdPosLds;  // block-uniform
+  if (staged) {
+    stage_positions<true>(a.pos16 + ra0, cnt0, spos);
+    stage_positions<true>(a.pos16 + ra1, cnt1, spos + cnt0 * PER);
+  }
+  if (wave == 0) {
+    int len = 0;
+    bool any_long = false;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int le = __shfl_down(la[p], 1);
+      any_long = any_long || long_segment(la[p], le, a.long_period);
+      len += le - la[p];
+      if (lane <= kBwdFeat) s_seg[p][lane] = la[p];
+    }
+    rank_features(lane < nf && !any_long ? len : 0, lane, s_perm);
+  }
+  __syncthreads();
+
+  const int g = lane / TCH, t = lane % TCH;
+  const int f32 = s_perm[wave * (kWave / TCH) + g];
+  const int s0 = s_seg[0][f32], s1 = s_seg[0][f32 + 1], u0 = s_seg[1][f32], u1 = s_seg[1][f32 + 1];
+  const bool live = f32 < nf && !long_segment(s0, s1, a.long_period) && !long_segment(u0, u1, a.long_period);
+  const int n0 = live ? s1 - s0 : 0, n1 = live ? u1 - u0 : 0;
+  int min0, max0, min1, max1;
+  group_minmax<TCH>(n0, min0, max0);
+  group_minmax<TCH>(n1, min1, max1);
+  const int64_t f = fb + (f32 < nf ? f32 : 0);
+  const int blk = block_of(f, a.dst.n, a.dst.start);
+  f32x4 *drow = pick(a.dst.p, blk) + (f - pick(a.dst.start, blk)) * a.map.cols4;
+  const int t0 = it.tile * a.tile_group, t1 = min(t0 + a.tile_group, a.ntiles);
+  for (int tile = t0; tile < t1; ++tile) {  // workgroup-uniform
+    const int colm = tile_col(a.map, tile, t);
+    const char *g0 = reinterpret_cast<const char *>(a.gt + (int64_t)tile * a.B * TCH);
+    const char *g1 = reinterpret_cast<const char *>(a.gt1 + (int64_t)tile * a.B * TCH);
+    f32x4 d0 = f32x4{0.f, 0.f, 0.f, 0.f}, d1 = d0;
+    if (staged) {
+      bwd_list_sum<TCH>(spos + (s0 - ra0), n0, min0, max0, t, g0, d0);
+      bwd_list_sum<TCH>(spos + cnt0 * PER + (u0 - ra1), n1, min1, max1, t, g1, d1);
+    } else {
+      bwd_list_sum<TCH>(a.pos16 + s0, n0, min0, max0, t, g0, d0);
+      bwd_list_sum<TCH>(a.pos16 + u0, n1, min1, max1, t, g1, d1);
+    }
+    if (live && colm >= 0) store_row<NT>(drow + colm, d0 + d1);
+  }
+}
+
 // A batch whose whole grad tile fits an XCD's L2 (4 MB: B <= 32768) is gathered
 // in one position chunk: no partial weight grads to store and reload (B = 16384:
 // 0.768 -> 0.619 ms per step, B = 32768: 1.139 -> 0.998 ms).  At B = 65536 one
@@ -893,6 +1031,12 @@ __global__ __launch_bounds__(kBlock) void bwd_tiled_gather_kernel(TiledArgs a) {
 // 1048: 512 55 / 47, 1536 59 / 58;  517: even.
 bool few_slots(int64_t B, int K, int64_t N) {
   return B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) && B * (int64_t)K <= 4 * N;
+}
+
+// Long-segment slots per tile of a gather over so many slots: at most
+// slots / period segments are long, and an empty slot is a workgroup.
+int long_slots(int64_t slots, int period) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kLongSlots, slots / period));
 }
 
 // Tiles per workgroup of a one-chunk gather.  A feature block's segment bounds,
@@ -929,7 +1073,8 @@ struct BiasFinal {
 int launch_tiled_gather(bool nt, const int32_t *seg, const int32_t *pos, const uint16_t *pos16, int64_t chunk_base,
                         int64_t N, const f32x4 *gt, int64_t B, const ColMap &map, const RowDst &dst, f32x4 *tmp,
                         int src_mode, int dst_mode, int ntiles, int ngroups, const int32_t *long_list,
-                        const int *long_count, int nlong, hipStream_t s, const BiasFinal *bias = nullptr) {
+                        const int *long_count, int nlong, int long_period, hipStream_t s,
+                        const BiasFinal *bias = nullptr) {
   const bool one_chunk = src_mode == kSrcZero && dst_mode != kDstTmp;
   const int tg = one_chunk && pos16 != nullptr ? gather_tile_group(B, ntiles, ngroups) : 1;
   const int64_t items = tile_sched_items_per_xcd(ntiles, nlong) +
@@ -940,7 +1085,7 @@ int launch_tiled_gather(bool nt, const int32_t *seg, const int32_t *pos, const u
   const int64_t gblocks = items * kXcds;
   const TiledArgs a{seg, pos, pos16, (int)chunk_base, N, gt, B, map, dst, tmp, src_mode, dst_mode, ntiles, ngroups,
                     long_list, long_count, nlong, gblocks, bias ? bias->partial : nullptr, bias ? bias->nparts : 0,
-                    bias ? bias->cols : 0, bias ? bias->db : nullptr, bias ? bias->overwrite : 0, tg};
+                    bias ? bias->cols : 0, bias ? bias->db : nullptr, bias ? bias->overwrite : 0, tg, nullptr, long_period};
   const bool p16 = pos16 != nullptr;
   const dim3 grid((unsigned)(gblocks + (bias ? bias_final_blocks(bias->cols) : 0)));
   if (tg > 1)
@@ -951,6 +1096,26 @@ int launch_tiled_gather(bool nt, const int32_t *seg, const int32_t *pos, const u
                            : (p16 ? bwd_tiled_gather_kernel<false, true, false> : bwd_tiled_gather_kernel<false, false, false>)),
                        grid, dim3(kBlock), lds, s, a);
   return check_launch("tiled feature gather");
+}
+
+// Both perspectives' weight grads of a one-chunk batch (bwd_pair_gather_kernel).
+int launch_pair_gather(const SegBufs &sb, const int32_t *pos, int64_t N, const f32x4 *gt0, const f32x4 *gt1, int64_t B,
+                       int K, const ColMap &map, const RowDst &dst, const BiasFinal &bias, hipStream_t s) {
+  const int ntiles = map_tiles(map);
+  const int ngroups = (int)ceil_div(N, kBwdFeat);
+  const int tg = gather_tile_group(2 * B, ntiles, ngroups);
+  const int period = long_period(B, K, N), nlong = long_slots(2 * B * K, period);
+  const int64_t gblocks =
+      (tile_sched_items_per_xcd(ntiles, nlong) + tile_sched_items_per_xcd((int)ceil_div(ntiles, tg), ngroups)) * kXcds;
+  if ((uintptr_t)sb.pos16 % 16 != 0) return fail(SFT_EINVAL, "pair feature gather: sorted positions not 16-byte aligned");
+  const TiledArgs a{sb.seg, pos, sb.pos16, 0, N, gt0, B, map, dst, nullptr, kSrcZero, kDstOut, ntiles, ngroups,
+                    sb.list, sb.count, nlong, gblocks, bias.partial, bias.nparts, bias.cols, bias.db, bias.overwrite,
+                    tg, gt1, period};
+  const dim3 grid((unsigned)(gblocks + bias_final_blocks(bias.cols)));
+  const size_t lds = (size_t)gather_lds(kDstOut).bytes;
+  hipLaunchKernelGGL((B * kBwdTileCh * 16 >= kNtStoreTileBytes ? bwd_pair_gather_kernel<true> : bwd_pair_gather_kernel<false>),
+                     grid, dim3(kBlock), lds, s, a);
+  return check_launch("pair feature gather");
 }
 
 // dV[j, :] = sum over i < reps of dWb[i * period + j, :], i ascending (the
@@ -1150,13 +1315,21 @@ __global__ __launch_bounds__(kBlock) void zero_kernel(float *__restrict__ p, int
 template <typename T, int CPL>
 __global__ __launch_bounds__(kBlock) void bias_partial_kernel(const T *__restrict__ grad, int64_t B, int64_t cols,
                                                               int64_t rows_per_block, T *__restrict__ partial,
-                                                              T *__restrict__ gt, int gt_shift) {
+                                                              T *__restrict__ gt, int gt_shift,
+                                                              const T *__restrict__ grad1, T *__restrict__ gt1,
+                                                              int nparts) {
+  // workgroups from nparts on take the second grad (grad1 into gt1) likewise
+  const bool second = (int)blockIdx.x >= nparts;  // whole block: uniform
+  if (second) {
+    grad = grad1;
+    gt = gt1;
+  }
   constexpr int U = 4;
   __shared__ T red[kWavesPerBlock][kWave * CPL];
   const int wave = uniform(threadIdx.x / kWave);
   const int lane = threadIdx.x % kWave;
   const int64_t c0 = (int64_t)blockIdx.y * (kWave * CPL) + lane;
-  const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
+  const int64_t r0 = (int64_t)(blockIdx.x - (second ? nparts : 0)) * rows_per_block;
   const int64_t r1 = std::min<int64_t>(B, r0 + rows_per_block);
   bool colok[CPL];
   T acc[CPL];
@@ -1210,9 +1383,9 @@ __global__ __launch_bounds__(kBlock) void bias_final_kernel(const T *__restrict_
 
 template <typename T, int G, int CPL>
 void launch_gather(dim3 grid, hipStream_t s, const int32_t *seg_start, const int32_t *pos, int64_t N, const void *grad,
-                   int64_t cols, void *dW, int overwrite, const SegBufs &sb, int nlong) {
+                   int64_t cols, void *dW, int overwrite, const SegBufs &sb, int nlong, int period) {
   hipLaunchKernelGGL((gather_rows_kernel<T, G, CPL, 4>), grid, dim3(kBlock), 0, s, seg_start, pos, N,
-                     static_cast<const T *>(grad), cols, static_cast<T *>(dW), overwrite, sb.list, sb.count, nlong);
+                     static_cast<const T *>(grad), cols, static_cast<T *>(dW), overwrite, sb.list, sb.count, nlong, period);
 }
 
 #define SFT_CPL_CASES(FN, T, G, ...) \
@@ -1317,17 +1490,18 @@ int make_layout(int64_t B, int K, int64_t N, int L, uint32_t flags, BwdLayout &l
 }
 
 int launch_bias_partial(const float *grad, int64_t B, int L, int nparts, float *partial, f32x4 *gt, bool vec,
-                        hipStream_t s, int gt_tch = 8) {
-  // tile width in the kernel's element type: gt_tch 16-byte chunks, or 4 x as many floats
-  const int gt_shift = (gt_tch == 4 ? 2 : gt_tch == 16 ? 4 : 3) + (vec ? 0 : 2);
+                        hipStream_t s, const float *grad1 = nullptr, f32x4 *gt1 = nullptr) {
+  // tile width in the kernel's element type: 8 16-byte chunks, or 4 x as many floats
+  const int gt_shift = vec ? 3 : 5;
   const int64_t cols = vec ? L / 4 : L;
   const int64_t rows = ceil_div(std::max<int64_t>(B, 1), nparts);
   const int cpl = (int)std::min<int64_t>(ceil_div(cols, kWave), kMaxCpl);
-  const dim3 pgrid((unsigned)nparts, (unsigned)ceil_div(cols, (int64_t)kWave * cpl));
+  const dim3 pgrid((unsigned)(grad1 ? 2 * nparts : nparts), (unsigned)ceil_div(cols, (int64_t)kWave * cpl));
   ProfScope prof(kProfBwdBiasPartial, s);
 #define SFT_BIAS_CASE(T, C)                                                                                  \
   hipLaunchKernelGGL((bias_partial_kernel<T, C>), pgrid, dim3(kBlock), 0, s, reinterpret_cast<const T *>(grad), \
-                     B, cols, rows, reinterpret_cast<T *>(partial), reinterpret_cast<T *>(gt), gt_shift)
+                     B, cols, rows, reinterpret_cast<T *>(partial), reinterpret_cast<T *>(gt), gt_shift,              \
+                     reinterpret_cast<const T *>(grad1), reinterpret_cast<T *>(gt1), nparts)
 #define SFT_BIAS_SWITCH(T)               \
   switch (cpl) {                         \
     case 1: SFT_BIAS_CASE(T, 1); break;  \
@@ -1363,13 +1537,13 @@ int launch_bias_final(const float *partial, int nparts, int L, float *db, int ov
 
 // Segment starts of one sort and its lists of long segments (the counts
 // were zeroed by the sort).
-int launch_segments(const unsigned *keys, int64_t M, int nc, int64_t nfeat, const unsigned *totals, int ntot,
+int launch_segments(const unsigned *keys, int64_t M, int period, int nc, int64_t nfeat, const unsigned *totals, int ntot,
                     const SegBufs &sb, const int32_t *pos, int64_t chunk_rows, hipStream_t s) {
   ProfScope prof(kProfBwdOffsets, s);
   uint16_t *p16 = chunk_rows <= 65536 ? sb.pos16 : nullptr;
   hipLaunchKernelGGL(seg_offsets_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(M + 1, kBlock), kSegBlocks)),
                      dim3(kBlock), 0, s, keys, (int64_t)nc * nfeat, totals, ntot, sb.seg, nfeat, sb.list, sb.count,
-                     pos, p16, (int)std::min<int64_t>(chunk_rows, 65536));
+                     pos, p16, (int)std::min<int64_t>(chunk_rows, 65536), period);
   return check_launch("segment offsets");
 }
 
@@ -1437,7 +1611,7 @@ int sort_and_segments(const int32_t *idx, int64_t B, int K, int64_t N, int nc, v
   if (slot_sort_buckets_supported(N, nc)) {
     ProfScope prof(kProfBwdSort, s);
     return slot_sort_buckets(idx, M, K, N, (int)crow, nc, sort_ws, sb.seg, sb.list, sb.count,
-                             crow <= 65536 ? sb.pos16 : nullptr, kLongSeg, pos, s);
+                             crow <= 65536 ? sb.pos16 : nullptr, long_period(B, K, N), pos, s);
   }
   unsigned *keys = nullptr, *totals = nullptr;
   int ntot = 0, rc;
@@ -1446,7 +1620,7 @@ int sort_and_segments(const int32_t *idx, int64_t B, int K, int64_t N, int nc, v
     if ((rc = slot_sort(idx, M, K, N, (int)crow, nc, sort_ws, &keys, pos, &totals, &ntot, sb.count, nc, s)) != SFT_OK)
       return rc;
   }
-  return launch_segments(keys, M, nc, N, totals, ntot, sb, *pos, crow, s);
+  return launch_segments(keys, M, long_period(B, K, N), nc, N, totals, ntot, sb, *pos, crow, s);
 }
 
 }  // namespace
@@ -1496,6 +1670,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
   char *w = static_cast<char *>(ws);
   const int overwrite = (flags & SFT_BWD_OVERWRITE) ? 1 : 0;
   const int64_t M = B * K;
+  const int period = long_period(B, K, N);
 
   // The tiled weight-grad gather reads the grad in column tiles; the bias pass
   // writes that layout while it streams the grad (16-byte loads when the grad
@@ -1544,14 +1719,14 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
       if ((rc = check_launch("long-segment count clear")) != SFT_OK) return rc;
       const int nb0 = chunk0_split ? slot_sort_buckets_chunk0(N, nc) : 0;
       if ((rc = slot_sort_buckets_low(pw + pl.sort, M, N, (int)crow, nc, pos, sbs.seg, sbs.list, sbs.count,
-                                      crow <= 65536 ? sbs.pos16 : nullptr, kLongSeg, side, 0,
+                                      crow <= 65536 ? sbs.pos16 : nullptr, period, side, 0,
                                       nb0 > 0 ? nb0 : -1)) != SFT_OK)
         return rc;
       if (nb0 > 0) {
         if ((rc = mark_side(kChunk0Mark)) != SFT_OK) return rc;
         chunk0_marked = true;
         if ((rc = slot_sort_buckets_low(pw + pl.sort, M, N, (int)crow, nc, pos, sbs.seg, sbs.list, sbs.count,
-                                        crow <= 65536 ? sbs.pos16 : nullptr, kLongSeg, side, nb0, -1)) != SFT_OK)
+                                        crow <= 65536 ? sbs.pos16 : nullptr, period, side, nb0, -1)) != SFT_OK)
           return rc;
       }
     } else {
@@ -1570,8 +1745,8 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
   const bool fuse_bias_final = tiled && M > 0 && (L % 4 == 0) && ((uintptr_t)grad % 16 == 0) && ((uintptr_t)db % 16 == 0);
   {
     const bool vec = (L % 4 == 0) && ((uintptr_t)grad % 16 == 0) && ((uintptr_t)db % 16 == 0);
-    if ((rc = launch_bias_partial(grad, B, L, lay.nparts, reinterpret_cast<float *>(w + lay.partial), gt, vec, s,
-                                  kBwdTileCh)) != SFT_OK)
+    if ((rc = launch_bias_partial(grad, B, L, lay.nparts, reinterpret_cast<float *>(w + lay.partial), gt, vec, s)) !=
+        SFT_OK)
       return rc;
     // with the tiled gather, its first launch reduces the partials too
     if (!(fuse_bias_final && SFT_BWD_FUSE_BIAS_FINAL) &&
@@ -1648,7 +1823,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
       const int64_t crow = nc > 1 ? half_rows(B) : B;
       rc = launch_tiled_gather(nt, seg + (int64_t)h * N, pos, crow <= 65536 ? sb.pos16 : nullptr, h * crow, N, gt, B,
                                map, dst, tmp, h == 0 ? kSrcZero : kSrcTmp, h == nc - 1 ? kDstOut : kDstTmp, ntiles,
-                               ngroups, sb.list + h * N, sb.count + h, kLongSlots, s,
+                               ngroups, sb.list + h * N, sb.count + h, long_slots(M, period), period, s,
                                h == 0 && fuse_bias_final && SFT_BWD_FUSE_BIAS_FINAL ? &bf : nullptr);
       if (rc != SFT_OK) return rc;
     }
@@ -1659,14 +1834,14 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
     const int64_t cols = vec ? L / 4 : L;
     const Mapping m = choose_mapping(cols);
     const int fpb = kWavesPerBlock * (kWave / m.G);
-    // long segments hold more than kLongSeg slots each: at most M / kLongSeg of them
-    const int nlong = vec ? (int)std::min<int64_t>(kRowLongBlocks, M / kLongSeg * ceil_div(cols, (int64_t)8)) : 0;
+    // long segments hold more than `period` slots each: at most M / period of them
+    const int nlong = vec ? (int)std::min<int64_t>(kRowLongBlocks, M / period * ceil_div(cols, (int64_t)8)) : 0;
     const dim3 grid((unsigned)(nlong + ceil_div(N, fpb)), (unsigned)m.slabs);
     ProfScope prof(kProfBwdGather, s);
     if (vec) {
-      SFT_G_CASES(launch_gather, f32x4, grid, s, seg, pos, N, grad, cols, dW, overwrite, sb, nlong)
+      SFT_G_CASES(launch_gather, f32x4, grid, s, seg, pos, N, grad, cols, dW, overwrite, sb, nlong, period)
     } else {
-      SFT_G_CASES(launch_gather, float, grid, s, seg, pos, N, grad, cols, dW, overwrite, sb, 0)
+      SFT_G_CASES(launch_gather, float, grid, s, seg, pos, N, grad, cols, dW, overwrite, sb, 0, period)
     }
   }
   return check_launch("feature row gather");
@@ -1678,9 +1853,15 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
 // grad tiles (one perspective at a time) | tmp (sums between position chunks,
 // tile-major).
 struct PairLayout {
-  size_t partial, sort[2], seg[2], gt, tmp, total;
+  size_t partial, sort[2], seg[2], gt, gt1, tmp, total;
   int nparts, nc;
+  bool one_launch;  // one sort, one bias pass and one gather of both perspectives
 };
+
+// Batches whose two grad tiles fit an XCD's L2 together (B <= 16 384).
+bool pair_one_launch(int64_t B, int64_t N) {
+  return 2 * B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) && slot_sort_buckets_supported(N, 2);
+}
 
 void make_pair_layout(int64_t B, int K, int64_t N, int L, PairLayout &lay) {
   const int64_t M = B * K;
@@ -1689,6 +1870,19 @@ void make_pair_layout(int64_t B, int K, int64_t N, int L, PairLayout &lay) {
   size_t off = 0;
   lay.partial = off;
   off = align256(off + (size_t)2 * lay.nparts * (size_t)L * sizeof(float));
+  lay.one_launch = pair_one_launch(B, N);
+  if (lay.one_launch) {
+    lay.sort[0] = lay.sort[1] = off;
+    off = align256(off + slot_sort_workspace(std::max<int64_t>(2 * M, 1)));
+    lay.seg[0] = lay.seg[1] = off;
+    off = align256(off + seg_region_bytes(2, N, 2 * M));
+    lay.gt = off;
+    off = align256(off + (size_t)(ceil_div(L, 32) * B * 32) * sizeof(float));
+    lay.gt1 = off;
+    off = align256(off + (size_t)(ceil_div(L, 32) * B * 32) * sizeof(float));
+    lay.tmp = lay.total = off;
+    return;
+  }
   for (int p = 0; p < 2; ++p) {  // each perspective sorts into its own buffers
     lay.sort[p] = off;
     off = align256(off + slot_sort_workspace(std::max<int64_t>(M, 1)));
@@ -1697,7 +1891,7 @@ void make_pair_layout(int64_t B, int K, int64_t N, int L, PairLayout &lay) {
   }
   // grad tiles, one perspective at a time: perspective 1's bias pass writes
   // them after perspective 0's gathers have read theirs (same stream)
-  lay.gt = off;
+  lay.gt = lay.gt1 = off;
   off = align256(off + (size_t)(ceil_div(L, 32) * B * 32) * sizeof(float));
   lay.tmp = off;
   off = align256(off + (size_t)(ceil_div(L, 32) * N * 32) * sizeof(float));
@@ -1725,7 +1919,7 @@ static int pair_sort_perspective(const int32_t *idx, int64_t B, int K, int64_t N
   if (slot_sort_buckets_supported(N, nc)) {
     ProfScope prof(kProfBwdSort, s);
     return slot_sort_buckets(idx, M, K, N, (int)crow, nc, sort_ws, out.sb.seg, out.sb.list, out.sb.count,
-                             crow <= 65536 ? out.sb.pos16 : nullptr, kLongSeg, &out.pos, s);
+                             crow <= 65536 ? out.sb.pos16 : nullptr, long_period(B, K, N), &out.pos, s);
   }
   {
     ProfScope prof(kProfBwdSort, s);
@@ -1733,13 +1927,13 @@ static int pair_sort_perspective(const int32_t *idx, int64_t B, int K, int64_t N
                         s)) != SFT_OK)
       return rc;
   }
-  return launch_segments(keys, M, nc, N, totals, ntot, out.sb, out.pos, crow, s);
+  return launch_segments(keys, M, long_period(B, K, N), nc, N, totals, ntot, out.sb, out.pos, crow, s);
 }
 
 // One perspective's position-chunk launches of the tiled gather, the sums
 // carried between chunks in tmp: perspective 0's last launch stores its sums to
 // dst, perspective 1's adds them to dst.
-static int pair_gather_perspective(int p, const SortedSlots &ss, int64_t B, int64_t N, const ColMap &map,
+static int pair_gather_perspective(int p, const SortedSlots &ss, int64_t B, int K, int64_t N, const ColMap &map,
                                    const f32x4 *gt, const RowDst &dst, f32x4 *tmp, int nc, hipStream_t s,
                                    const BiasFinal *bias = nullptr) {  // reduced by the first launch
   const int ntiles = map_tiles(map);
@@ -1753,7 +1947,8 @@ static int pair_gather_perspective(int p, const SortedSlots &ss, int64_t B, int6
     const int64_t crow = nc > 1 ? half_rows(B) : B;
     const int rc = launch_tiled_gather(nt, ss.sb.seg + (int64_t)h * N, ss.pos, crow <= 65536 ? ss.sb.pos16 : nullptr,
                                        h * crow, N, gt, B, map, dst, tmp, src_mode,
-                                       dst_mode, ntiles, ngroups, ss.sb.list + h * N, ss.sb.count + h, kLongSlots, s,
+                                       dst_mode, ntiles, ngroups, ss.sb.list + h * N, ss.sb.count + h,
+                                       long_slots(B * K, long_period(B, K, N)), long_period(B, K, N), s,
                                        h == 0 ? bias : nullptr);
     if (rc != SFT_OK) return rc;
   }
@@ -1777,6 +1972,23 @@ static int pair_sort_both(const int32_t *idx0, const int32_t *idx1, int64_t B, i
     if ((rc = mark_side(p)) != SFT_OK) return rc;
   }
   side_join.release();  // the caller waits for each mark before that perspective's gathers
+  return SFT_OK;
+}
+
+// Both perspectives' slots in one sort on the side stream (key = perspective N +
+// feature, positions of perspective 1 from B on); joined by the caller.
+static int pair_sort_once(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, int64_t N, char *sort_ws,
+                          int32_t *seg, SortedSlots &out, hipStream_t s) {
+  hipStream_t side;
+  int rc = fork_side(s, &side);
+  if (rc != SFT_OK) return rc;
+  SideJoinGuard side_join(s);
+  out.sb = seg_bufs(seg, 2, N);
+  ProfScope prof(kProfBwdSort, side);
+  if ((rc = slot_sort_buckets(idx0, 2 * B * K, K, N, (int)B, 2, sort_ws, out.sb.seg, out.sb.list, out.sb.count,
+                              out.sb.pos16, long_period(B, K, N), &out.pos, side, idx1)) != SFT_OK)
+    return rc;
+  side_join.release();
   return SFT_OK;
 }
 
@@ -1809,24 +2021,39 @@ int bwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, con
   f32x4 *gt = reinterpret_cast<f32x4 *>(w + lay.gt);
   f32x4 *tmp = reinterpret_cast<f32x4 *>(w + lay.tmp);
   SortedSlots ss[2];
-  int rc = pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s);
-  if (rc != SFT_OK) return rc;
+  // the bias reduction over both perspectives' partials rides in perspective
+  // 1's first gather launch
+  const BiasFinal bf{reinterpret_cast<const f32x4 *>(partial), 2 * lay.nparts, L / 4, reinterpret_cast<f32x4 *>(db), 1};
+  int rc;
+  if (lay.one_launch) {
+    f32x4 *gt1 = reinterpret_cast<f32x4 *>(w + lay.gt1);
+    if ((rc = pair_sort_once(idx0, idx1, B, K, N, w + lay.sort[0], reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0],
+                             s)) != SFT_OK)
+      return rc;
+    SideJoinGuard side_join(s);
+    if ((rc = launch_bias_partial(grad0, B, L, lay.nparts, partial, gt, true, s, grad1, gt1)) != SFT_OK) return rc;
+    side_join.release();
+    if ((rc = join_side(s)) != SFT_OK) return rc;
+    {
+      ProfScope prof(kProfBwdTiled, s);
+      if ((rc = launch_pair_gather(ss[0].sb, ss[0].pos, N, gt, gt1, B, K, map, dst, bf, s)) != SFT_OK) return rc;
+    }
+    return virtual_reduce(vgrad_src, vgrad, vperiod, vreps, nvirt, L / 4, s);
+  }
+  if ((rc = pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s)) != SFT_OK) return rc;
   SideJoinGuard side_join(s);  // until both marks are waited for
   // Each perspective's bias pass (which also writes its grad tiles) right
   // before its gathers, the sorts on the side stream meanwhile: both bias
   // passes first, beside both sorts, took 133 against 107 us each (composed
   // HalfKAv2_hm^ step 1.752 -> 1.740 ms, Full_Threats+HalfKAv2_hm^ 6.988 ->
   // 6.951 ms).
-  // the bias reduction over both perspectives' partials rides in perspective
-  // 1's first gather launch
-  const BiasFinal bf{reinterpret_cast<const f32x4 *>(partial), 2 * lay.nparts, L / 4, reinterpret_cast<f32x4 *>(db), 1};
   for (int p = 0; p < 2; ++p) {
     const float *grad = p == 0 ? grad0 : grad1;
     if ((rc = launch_bias_partial(grad, B, L, lay.nparts, partial + (size_t)p * lay.nparts * L, gt, true, s)) !=
         SFT_OK)
       return rc;
     if ((rc = wait_side(s, p)) != SFT_OK) return rc;
-    if ((rc = pair_gather_perspective(p, ss[p], B, N, map, gt, dst, tmp, lay.nc, s,
+    if ((rc = pair_gather_perspective(p, ss[p], B, K, N, map, gt, dst, tmp, lay.nc, s,
                                       p == 1 && SFT_BWD_FUSE_BIAS_FINAL ? &bf : nullptr)) != SFT_OK)
       return rc;
   }
@@ -1842,6 +2069,7 @@ int bwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, con
 struct TransformLayout {
   size_t partial, sort[2], seg[2], gt0, gt1, tmp, total;
   int nparts, nc;
+  bool one_launch;
 };
 
 void make_transform_layout(int64_t B, int K, int64_t N, int L, int L1, TransformLayout &lay) {
@@ -1853,18 +2081,20 @@ void make_transform_layout(int64_t B, int K, int64_t N, int L, int L1, Transform
   size_t off = 0;
   lay.partial = off;
   off = align256(off + (size_t)lay.nparts * (size_t)L * sizeof(float));
-  for (int p = 0; p < 2; ++p) {
+  lay.one_launch = pair_one_launch(B, N);
+  for (int p = 0; p < (lay.one_launch ? 1 : 2); ++p) {
+    const int64_t slots = lay.one_launch ? 2 * M : M;
     lay.sort[p] = off;
-    off = align256(off + slot_sort_workspace(std::max<int64_t>(M, 1)));
+    off = align256(off + slot_sort_workspace(std::max<int64_t>(slots, 1)));
     lay.seg[p] = off;
-    off = align256(off + seg_region_bytes(lay.nc, N, M));
+    off = align256(off + seg_region_bytes(lay.one_launch ? 2 : lay.nc, N, slots));
   }
   lay.gt0 = off;
   off = align256(off + gtb);
   lay.gt1 = off;
   off = align256(off + gtb);
   lay.tmp = off;
-  off = align256(off + (size_t)map_tiles(map) * (size_t)N * 128);
+  if (!lay.one_launch) off = align256(off + (size_t)map_tiles(map) * (size_t)N * 128);
   lay.total = off;
 }
 
@@ -1901,9 +2131,11 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   e.partial = reinterpret_cast<f32x4 *>(w + lay.partial);
   e.P = L - L1;
   SortedSlots ss[2];  // sorted on the side stream while the epilogue runs
-  int rc = pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s);
+  int rc = lay.one_launch ? pair_sort_once(idx0, idx1, B, K, N, w + lay.sort[0],
+                                           reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], s)
+                          : pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s);
   if (rc != SFT_OK) return rc;
-  SideJoinGuard side_join(s);  // until both marks are waited for
+  SideJoinGuard side_join(s);  // until the side stream's marks are waited for
   {
     ProfScope prof(kProfBwdEpilogue, s);
     hipLaunchKernelGGL(bwd_epilogue_kernel, dim3((unsigned)lay.nparts), dim3(kBlock), 0, s, e, map, B,
@@ -1913,6 +2145,16 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   // the bias reduction rides in perspective 0's first gather launch
   const BiasFinal bf{reinterpret_cast<const f32x4 *>(w + lay.partial), lay.nparts, L / 4,
                      reinterpret_cast<f32x4 *>(db), 1};
+  if (lay.one_launch) {
+    side_join.release();
+    if ((rc = join_side(s)) != SFT_OK) return rc;
+    {
+      ProfScope prof(kProfBwdTiled, s);
+      if ((rc = launch_pair_gather(ss[0].sb, ss[0].pos, N, gt0, gt1, B, K, map, dst, bf, s)) != SFT_OK)
+        return rc;
+    }
+    return virtual_reduce(vgrad_src, vgrad, vperiod, vreps, nvirt, L / 4, s);
+  }
   if (!SFT_BWD_FUSE_BIAS_FINAL &&
       (rc = launch_bias_final(reinterpret_cast<const float *>(w + lay.partial), lay.nparts, L, db, 1, true, s)) !=
           SFT_OK)
@@ -1920,7 +2162,7 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   f32x4 *tmp = reinterpret_cast<f32x4 *>(w + lay.tmp);
   for (int p = 0; p < 2; ++p) {
     if ((rc = wait_side(s, p)) != SFT_OK) return rc;
-    if ((rc = pair_gather_perspective(p, ss[p], B, N, map, p == 0 ? gt0 : gt1, dst, tmp, lay.nc, s,
+    if ((rc = pair_gather_perspective(p, ss[p], B, K, N, map, p == 0 ? gt0 : gt1, dst, tmp, lay.nc, s,
                                       p == 0 && SFT_BWD_FUSE_BIAS_FINAL ? &bf : nullptr)) != SFT_OK)
       return rc;
   }

@@ -46,12 +46,17 @@ constexpr int kMaxRadix = 1024;  // 10-bit digits (the bucket sort's first pass)
 
 // Key of slot s (s < 2^31): chunk(b) * N + feature for an active slot, the
 // sentinel (>= every real key) for an inactive one; the value is b = s / K.
+// Slots from M0 on are idx1's (two perspectives sorted at once: chunk_rows = B
+// makes the perspective the chunk); one matrix passes itself and all its slots.
 struct SlotKey {
-  const int32_t *idx;
+  const int32_t *idx, *idx1;
+  int64_t M0;
   unsigned N;
   FastDiv divK, divChunk;
   unsigned sentinel;
-  __device__ __forceinline__ unsigned key(int64_t s) const { return key_of(s, (unsigned)idx[s]); }
+  __device__ __forceinline__ unsigned load(int64_t s) const {
+    return (unsigned)(s < M0 ? idx : idx1 - M0)[s];
+  }
   // The key of slot s from its loaded index value v (loads issued apart from
   // the arithmetic, whose divisor checks are branches the loads do not cross).
   __device__ __forceinline__ unsigned key_of(int64_t s, unsigned v) const {
@@ -115,7 +120,7 @@ __global__ __launch_bounds__(kBlock) void radix_upsweep(SlotKey sk, const unsign
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       const int64_t e = std::min<int64_t>(base + (int64_t)i * kBlock + tid, count - 1);
-      k[i] = FIRST ? (unsigned)sk.idx[e] : kin[e];
+      k[i] = FIRST ? sk.load(e) : kin[e];
     }
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
@@ -289,7 +294,7 @@ __global__ __launch_bounds__(kBlock) void radix_downsweep(SlotKey sk, const unsi
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
     const int64_t ec = std::min<int64_t>(base + (int64_t)i * kWave + lane, last);
-    key[i] = FIRST ? (unsigned)sk.idx[ec] : kin[ec];
+    key[i] = FIRST ? sk.load(ec) : kin[ec];
     if (!FIRST) val[i] = vin[ec];
   }
 #pragma unroll
@@ -625,7 +630,7 @@ int slot_sort(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, i
   unsigned *hist = reinterpret_cast<unsigned *>(w + 4 * a);
   unsigned *totals = reinterpret_cast<unsigned *>(w + 4 * a + align256((size_t)(kMaxRadix * max_tiles) * 4));
   const unsigned nkeys = (unsigned)((int64_t)nchunks * N);
-  const SlotKey sk{idx, (unsigned)N, FastDiv((uint32_t)K), FastDiv((uint32_t)chunk_rows), nkeys};
+  const SlotKey sk{idx, idx, M, (unsigned)N, FastDiv((uint32_t)K), FastDiv((uint32_t)chunk_rows), nkeys};
   int rb, passes;
   sort_passes(nkeys, rb, passes);
   int rc;
@@ -690,13 +695,15 @@ static int bucket_bufs(void *ws, int64_t M, int64_t N, int nchunks, BucketBufs &
 
 // First half of the bucket sort: the radix pass on the high key bits, into
 // the workspace; zeroes clear[0 .. nclear) (stream-ordered).
+// idx1: the slots from M / 2 on (null: idx holds all M).
 int slot_sort_buckets_high(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, int nchunks, void *ws,
-                           int *clear, int nclear, hipStream_t s) {
+                           int *clear, int nclear, hipStream_t s, const int32_t *idx1) {
   BucketBufs bb;
   int rc = bucket_bufs(ws, M, N, nchunks, bb);
   if (rc != SFT_OK) return rc;
   const unsigned nkeys = (unsigned)((int64_t)nchunks * N);
-  const SlotKey sk{idx, (unsigned)N, FastDiv((uint32_t)K), FastDiv((uint32_t)chunk_rows), nkeys};
+  const SlotKey sk{idx, idx1 ? idx1 : idx, idx1 ? M / 2 : M, (unsigned)N, FastDiv((uint32_t)K),
+                   FastDiv((uint32_t)chunk_rows), nkeys};
 #define SFT_HIGH_PASS(RB)                                                                                          \
   rc = bb.big ? run_high_pass<RB, kSortItemsBig>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles, clear, \
                                                  nclear, s)                                                        \
@@ -753,11 +760,12 @@ int slot_sort_buckets_chunk0(int64_t N, int nchunks) {
 // counts zeroed by the first half.  Same results as slot_sort + the segment kernel.
 int slot_sort_buckets(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, int nchunks, void *ws,
                       int32_t *seg, int32_t *list, int *count, uint16_t *pos16, int long_period, int **pos_sorted,
-                      hipStream_t s) {
+                      hipStream_t s, const int32_t *idx1) {
   BucketBufs bb;
   int rc = bucket_bufs(ws, M, N, nchunks, bb);
   if (rc != SFT_OK) return rc;
-  if ((rc = slot_sort_buckets_high(idx, M, K, N, chunk_rows, nchunks, ws, count, nchunks, s)) != SFT_OK) return rc;
+  if ((rc = slot_sort_buckets_high(idx, M, K, N, chunk_rows, nchunks, ws, count, nchunks, s, idx1)) != SFT_OK)
+    return rc;
   if ((rc = slot_sort_buckets_low(ws, M, N, chunk_rows, nchunks, bb.v2, seg, list, count, pos16, long_period, s, 0,
                                   -1)) != SFT_OK)
     return rc;

@@ -47,11 +47,14 @@ SHAPES = [
     (3, 1000, 32, 1048, 16, 32, [(2000, 0)]),           # no virtual rows
     (4, 257, 24, 260, 0, 24, [(960, 32), (500, 0), (64, 16), (100, 0)]),  # four blocks, partial last tile
     (5, 2048, 160, 1048, 32, 160, [(6072, 0), (3072, 768)]),  # threats-shaped composition
+    (9, 5003, 32, 1048, 0, 32, [(24576, 768)]),  # one launch for both perspectives, two tiles a workgroup
+    (10, 16384, 8, 264, 0, 8, [(3072, 96), (700, 0)]),  # its largest batch, one tile a workgroup, skewed
+    (11, 16385, 8, 264, 0, 8, [(3072, 96), (700, 0)]),  # a launch per perspective, one position chunk, skewed
     (6, 6000, 32, 520, 16, 32, [(40, 8), (24, 0)]),  # 64 rows, one position chunk: every segment long
     (7, 40000, 32, 520, 16, 32, [(40, 8), (24, 0)]),  # two position chunks: long segments in both
     (8, 40000, 32, 520, 16, 32, [(3072, 96), (700, 0)]),  # two chunks, Zipf-skewed: hot and short segments
 ]
-ZIPF = {8: 1.0}  # seeds whose rows draw features with skewed frequencies
+ZIPF = {8: 1.0, 9: 0.7, 10: 1.0, 11: 1.0}  # seeds whose rows draw features with skewed frequencies
 
 
 def _indices(g, seed, B, N, K, lo, hi, sort):
