@@ -53,6 +53,37 @@ def test_encode_random(name, B, seed):
     _check(boards, stm, name)
 
 
+@pytest.mark.parametrize("name", ["HalfKAv2_hm", "Full_Threats+HalfKAv2_hm"])
+def test_encode_crowded_boards(name):
+    """Boards around and above 32 pieces (up to all 64 squares), rows past their caps
+    and several kings of a colour; 1 to 20 positions a wave."""
+    announce(f"encode crowded {name}")
+    g = np.random.default_rng(12)
+    for B in (1, 5, 700, 163840):
+        boards = np.full((B, 64), positions.EMPTY, np.uint8)
+        n = min(B, 700)
+        for b in range(n):
+            k = int(g.choice([30, 31, 32, 33, 34, 50, 64]))
+            sq = g.permutation(64)[:k]
+            boards[b, sq] = g.integers(0, 12 if b % 3 == 0 else 10, k)
+            back = (boards[b] < 2) & ((np.arange(64) < 8) | (np.arange(64) >= 56))
+            boards[b, back] += 2  # no pawns on the back ranks
+            boards[b, sq[0]], boards[b, sq[1]] = 10, 11
+        boards[n:] = boards[np.arange(B - n) % n]
+        stm = g.integers(0, 2, B).astype(np.uint8)
+        ref = fo.encode(boards, stm, SETS[name])
+        got = encode_batch(torch.from_numpy(boards).to(DEV), torch.from_numpy(stm).to(DEV), name, with_counts=True)
+        pieces = (boards < 12).sum(axis=1)
+        for key, cnt in (("white", "count_w"), ("black", "count_b")):
+            assert np.array_equal(host(got[key]), ref[key])
+            # counts: every feature, also those past the rows' caps (the oracle counts up to them)
+            whole = (pieces <= 32) & (ref[cnt] - np.minimum(pieces, 32) < 128)
+            assert np.array_equal(host(got[key + "_count"])[whole], ref[cnt][whole])
+            assert (host(got[key + "_count"]) >= ref[cnt]).all()
+        assert np.array_equal(host(got["us"]).reshape(-1), ref["us"])
+        assert np.array_equal(host(got["psqt_indices"]), (pieces - 1) // 4)
+
+
 def test_encode_threat_order_matches_the_reference_loops():
     """The GPU encoder's Full_Threats rows against the loop-order restatement
     (tests/threat_order.py), independently of the oracle's own walk."""
