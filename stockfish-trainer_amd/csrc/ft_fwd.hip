@@ -1246,12 +1246,28 @@ __global__ __launch_bounds__(kBlock) void i16_relayout_kernel(const i16x8 *__res
 }
 
 // --------------------------------------------------------------- quantize ----
+__device__ __forceinline__ short quantize_one(float x, float scale) {
+  const float r = __builtin_rintf(x * scale);  // binary32 product, round half to even
+  return (short)fminf(fmaxf(r, -32768.0f), 32767.0f);
+}
 __global__ __launch_bounds__(kBlock) void quantize_i16_kernel(const float *__restrict__ x, int64_t n, float scale,
                                                               int16_t *__restrict__ out) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-    float r = __builtin_rintf(x[i] * scale);  // binary32 product, round half to even
-    r = fminf(fmaxf(r, -32768.0f), 32767.0f);
-    out[i] = (int16_t)r;
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
+    out[i] = quantize_one(x[i], scale);
+}
+// The same for n8 runs of 8 values (16-byte aligned x and out): 16-byte loads
+// and stores.  23.4 M values (141 MB moved): 31.8 -> 24.1 us.
+__global__ __launch_bounds__(kBlock) void quantize_i16x8_kernel(const f32x4 *__restrict__ x, int64_t n8, float scale,
+                                                                i16x8 *__restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n8; i += (int64_t)gridDim.x * kBlock) {
+    const f32x4 a = __builtin_nontemporal_load(x + 2 * i), b = __builtin_nontemporal_load(x + 2 * i + 1);
+    i16x8 q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      q[e] = quantize_one(a[e], scale);
+      q[4 + e] = quantize_one(b[e], scale);
+    }
+    out[i] = q;
   }
 }
 
@@ -1846,9 +1862,15 @@ int fwd_i16(const int32_t *idx, int64_t B, int K, const int16_t *W, int64_t N, i
 
 int quantize_i16(const float *x, int64_t n, float scale, int16_t *out, hipStream_t s) {
   if (n == 0) return SFT_OK;
-  const int64_t blocks = std::min<int64_t>(ceil_div(n, kBlock), 1 << 16);
+  const bool vec = (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const int64_t n8 = vec ? n / 8 : 0, rest = n - 8 * n8;
+  auto blocks = [](int64_t items) { return dim3((unsigned)std::min<int64_t>(ceil_div(items, kBlock), 1 << 16)); };
   ProfScope prof(kProfQuantize, s);
-  hipLaunchKernelGGL(quantize_i16_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, x, n, scale, out);
+  if (n8 > 0)
+    hipLaunchKernelGGL(quantize_i16x8_kernel, blocks(n8), dim3(kBlock), 0, s, reinterpret_cast<const f32x4 *>(x), n8,
+                       scale, reinterpret_cast<i16x8 *>(out));
+  if (rest > 0)
+    hipLaunchKernelGGL(quantize_i16_kernel, blocks(rest), dim3(kBlock), 0, s, x + 8 * n8, rest, scale, out + 8 * n8);
   return check_launch("sft_quantize_i16");
 }
 

@@ -720,7 +720,7 @@ def leb128_encode(values: torch.Tensor) -> torch.Tensor:
     cap = n * {1: 2, 2: 3, 4: 5}[elem]
     dev = values.device
     out = torch.empty(max(cap, 1), dtype=torch.uint8, device=dev)
-    out_len = torch.zeros(1, dtype=torch.int64, device=dev)
+    out_len = torch.empty(1, dtype=torch.int64, device=dev)  # written by every call
     nb = ctypes.c_size_t(0)
     _check(lib().sft_leb128_workspace_size(n, ctypes.byref(nb)), "sft_leb128_workspace_size")
     ws, ptr = _workspace(int(nb.value), dev)

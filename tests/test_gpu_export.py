@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from gpu_helpers import DEV, announce, dev, host
+from oracle import ft_oracle
 from oracle import leb128_oracle as leb
 from sft_amd import _native
 from src.model.modules.features import get_feature_cls
@@ -31,6 +32,43 @@ def test_leb128_matches_oracle(dtype, n):
     a[:min(n, len(LIMITS[dtype]))] = LIMITS[dtype][:min(n, len(LIMITS[dtype]))]
     got = host(_native.leb128_encode(dev(a))).tobytes()
     assert got == leb.encode(a)
+
+
+# tiles of 4096 values, groups of 4 tiles; views off the 16-byte alignment
+@pytest.mark.parametrize("dtype", [np.int8, np.int16, np.int32])
+@pytest.mark.parametrize("n", [15, 16, 17, 4095, 4096, 16383, 16384, 16385, 40961])
+@pytest.mark.parametrize("skip", [0, 1, 3])
+def test_leb128_tile_edges(dtype, n, skip):
+    announce(f"leb128 edges {dtype.__name__} n={n} skip={skip}")
+    g = np.random.default_rng(n + skip)
+    info = np.iinfo(dtype)
+    a = (g.integers(info.min, info.max + 1, n + skip) >> g.integers(0, 8 * info.dtype.itemsize, n + skip)).astype(dtype)
+    assert host(_native.leb128_encode(dev(a)[skip:])).tobytes() == leb.encode(a[skip:])
+
+
+def test_leb128_scanned_groups():
+    """More groups than a writing workgroup sums itself (8192 of 16 384 values)."""
+    announce("leb128 scanned groups")
+    n = 8192 * 16384 + 5
+    a = torch.randint(-64, 64, (n,), dtype=torch.int8, device=DEV)  # codes of one byte
+    a[7], a[n - 2] = 100, -100                                       # and two of two
+    got = _native.leb128_encode(a)
+    assert got.numel() == n + 2
+    one = a & 0x7F
+    assert torch.equal(got[:7].to(torch.int8), one[:7]) and host(got[7:9]).tobytes() == bytes([0xE4, 0x00])
+    assert torch.equal(got[9:n - 1].to(torch.int8), one[8:n - 2])
+    assert host(got[n - 1:n + 1]).tobytes() == bytes([0x9C, 0x7F]) and int(got[-1]) == int(one[-1])
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 2049, 100003])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_quantize_run_edges(n, skip):
+    announce(f"quantize n={n} skip={skip}")
+    g = np.random.default_rng(n)
+    x = (g.standard_normal(n + skip) * 200).astype(np.float32)
+    x[-1] = np.float32(0.5 / 255.0)
+    got = host(_native.quantize_i16(dev(x)[skip:], 255.0))
+    assert np.array_equal(got, ft_oracle.quantize_i16(x[skip:], 255.0))
 
 
 def test_leb128_empty():
