@@ -42,6 +42,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
 int bwd_prep_bytes(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *bytes);
 int bwd_prepare(const int32_t *idx, int64_t B, int K, int64_t N, int L, uint32_t flags, void *prep,
                 size_t prep_bytes, hipStream_t s);
+bool sort_small(int64_t B, int K, int L);
 size_t index_lds_bytes(int G, int K);
 int fwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, const FoldSrc &src, int64_t N, int L,
                  const float *bias, float *out0, float *out1, void *ws, size_t ws_bytes, hipStream_t s);
@@ -119,9 +120,13 @@ SideState *side_state(bool create) {
   }
   if (!t_side[dev] && create) {
     auto st = std::make_unique<SideState>();
+    // The events order streams of one device only, so they need no system-scope
+    // fence (which writes the caches back): a step of four forks and joins
+    // 597 -> 588 us at B = 16384, L = 1048, 1704 -> 1694 us at B = 65536.
+    constexpr unsigned flags = hipEventDisableTiming | hipEventDisableSystemFence;
     bool ok = hipStreamCreateWithFlags(&st->stream, hipStreamNonBlocking) == hipSuccess &&
-              hipEventCreateWithFlags(&st->fork, hipEventDisableTiming) == hipSuccess;
-    for (hipEvent_t &e : st->mark) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+              hipEventCreateWithFlags(&st->fork, flags) == hipSuccess;
+    for (hipEvent_t &e : st->mark) ok = ok && hipEventCreateWithFlags(&e, flags) == hipSuccess;
     if (!ok) return nullptr;
     t_side[dev] = std::move(st);
   }
@@ -135,6 +140,17 @@ int fork_side(hipStream_t s, hipStream_t *side) {
   if (hipEventRecord(st->fork, s) != hipSuccess || hipStreamWaitEvent(st->stream, st->fork, 0) != hipSuccess)
     return fail(SFT_EHIP, "side stream: fork failed");
   *side = st->stream;
+  return SFT_OK;
+}
+
+int fork_sort(hipStream_t s, bool small, hipStream_t *side, bool *forked) {
+  *forked = !small;
+  if (small) {  // a captured fork costs the host nothing when it is replayed
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    *forked = hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
+  }
+  if (*forked) return fork_side(s, side);
+  *side = s;
   return SFT_OK;
 }
 
@@ -398,9 +414,11 @@ int sft_ft_fwd_f32_prep(const int32_t *idx, int64_t batch, int32_t max_active, c
     return sft_ft_fwd_f32_ex(idx, batch, max_active, weight, num_inputs, output_size, bias, out, workspace,
                              workspace_bytes, flags, stream);
   hipStream_t side;
-  int rc = fork_side(s, &side);
+  bool forked;
+  int rc = fork_sort(s, sort_small(batch, max_active, output_size), &side, &forked);
   if (rc != SFT_OK) return rc;
   SideJoinGuard side_join(s);
+  if (!forked) side_join.release();
   if ((rc = bwd_prepare(idx, batch, max_active, num_inputs, output_size, bwd_flags, prep, prep_bytes, side)) != SFT_OK)
     return rc;
   const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
@@ -412,7 +430,7 @@ int sft_ft_fwd_f32_prep(const int32_t *idx, int64_t batch, int32_t max_active, c
              : fwd_f32(idx, batch, max_active, weight, num_inputs, output_size, bias, out, s);
   if (rc != SFT_OK) return rc;
   side_join.release();
-  return join_side(s);
+  return forked ? join_side(s) : SFT_OK;
 }
 
 int sft_ft_bwd_f32_prepared(const int32_t *idx, int64_t batch, int32_t max_active, const float *grad_out,

@@ -28,6 +28,7 @@
 
 namespace sft {
 
+bool sort_small(int64_t B, int K, int L);
 size_t index_lds_bytes(int G, int K);
 size_t slot_sort_workspace(int64_t M);
 // Stable sort of the active slots by (position chunk, feature); also zeroes
@@ -1584,6 +1585,7 @@ bool prep_pays(int64_t B, int K, int L, uint32_t flags) {
 #ifndef SFT_BWD_SPLIT_BUCKETS
 #define SFT_BWD_SPLIT_BUCKETS 1
 #endif
+constexpr int64_t kSmallSort = 1 << 16, kSmallSortNarrow = 1 << 21;  // slots (sort_small)
 constexpr int kChunk0Mark = 1;  // side-stream mark after chunk 0's buckets
 bool prep_split(int64_t B, int K, int64_t N, int L, uint32_t flags) {
   return prep_pays(B, K, L, flags) && (int64_t)K * SFT_BWD_SPLIT_K_PER_L >= L &&
@@ -1624,6 +1626,16 @@ int sort_and_segments(const int32_t *idx, int64_t B, int K, int64_t N, int nc, v
 }
 
 }  // namespace
+
+// Whether a perspective's sort runs on the caller's stream: a fork and join
+// take about 27 us on the host, and a step whose launches take the host longer
+// than the GPU gains more from saving them than from the overlap.  Steps of both
+// perspectives launched eagerly, forked / in line, us: L = 1048 (N = 23 232), B = 300
+// 358 / 184, B = 2048 351 / 280, B = 4096 397 / 408; narrow rows (the split
+// prepared sort's), L = 136, B = 8192 417 / 271, B = 65 536 471 / 385.
+bool sort_small(int64_t B, int K, int L) {
+  return B * K <= ((int64_t)K * SFT_BWD_SPLIT_K_PER_L >= L ? kSmallSortNarrow : kSmallSort);
+}
 
 int bwd_prep_bytes(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *bytes) {
   PrepLayout p;
@@ -1708,8 +1720,9 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
       // the buckets on the side stream, beside the bias pass, from the radix
       // pass the forward left in the prepared buffer, into the workspace
       hipStream_t side;
-      if ((rc = fork_side(s, &side)) != SFT_OK) return rc;
-      side_join.emplace(s);
+      bool forked;
+      if ((rc = fork_sort(s, sort_small(B, K, L), &side, &forked)) != SFT_OK) return rc;
+      if (forked) side_join.emplace(s);
       const SegBufs sbs = seg_bufs(seg, nc, N);
       const int64_t crow = nc > 1 ? half_rows(B) : B;
       pos = reinterpret_cast<int32_t *>(w + lay.spos);
@@ -1717,7 +1730,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
       hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(kBlock), 0, side, reinterpret_cast<float *>(sbs.count),
                          (int64_t)nc);  // the long-segment counts (the forward's radix pass left them alone)
       if ((rc = check_launch("long-segment count clear")) != SFT_OK) return rc;
-      const int nb0 = chunk0_split ? slot_sort_buckets_chunk0(N, nc) : 0;
+      const int nb0 = chunk0_split && forked ? slot_sort_buckets_chunk0(N, nc) : 0;
       if ((rc = slot_sort_buckets_low(pw + pl.sort, M, N, (int)crow, nc, pos, sbs.seg, sbs.list, sbs.count,
                                       crow <= 65536 ? sbs.pos16 : nullptr, period, side, 0,
                                       nb0 > 0 ? nb0 : -1)) != SFT_OK)
@@ -1735,8 +1748,9 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
     }
   } else if (sorted) {
     hipStream_t side;
-    if ((rc = fork_side(s, &side)) != SFT_OK) return rc;
-    side_join.emplace(s);
+    bool forked;
+    if ((rc = fork_sort(s, sort_small(B, K, L), &side, &forked)) != SFT_OK) return rc;
+    if (forked) side_join.emplace(s);
     if ((rc = sort_and_segments(idx, B, K, N, nc, w + lay.sort, seg, &pos, side)) != SFT_OK) return rc;
   }
   const SegBufs sb = seg_bufs(seg, nc, N);
@@ -1976,13 +1990,15 @@ static int pair_sort_both(const int32_t *idx0, const int32_t *idx1, int64_t B, i
 }
 
 // Both perspectives' slots in one sort on the side stream (key = perspective N +
-// feature, positions of perspective 1 from B on); joined by the caller.
+// feature, positions of perspective 1 from B on); joined by the caller when
+// *forked.
 static int pair_sort_once(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, int64_t N, char *sort_ws,
-                          int32_t *seg, SortedSlots &out, hipStream_t s) {
+                          int32_t *seg, SortedSlots &out, bool *forked, hipStream_t s) {
   hipStream_t side;
-  int rc = fork_side(s, &side);
+  int rc = fork_sort(s, 2 * B * K <= 2 * kSmallSort, &side, forked);
   if (rc != SFT_OK) return rc;
   SideJoinGuard side_join(s);
+  if (!*forked) side_join.release();
   out.sb = seg_bufs(seg, 2, N);
   ProfScope prof(kProfBwdSort, side);
   if ((rc = slot_sort_buckets(idx0, 2 * B * K, K, N, (int)B, 2, sort_ws, out.sb.seg, out.sb.list, out.sb.count,
@@ -2027,13 +2043,15 @@ int bwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, con
   int rc;
   if (lay.one_launch) {
     f32x4 *gt1 = reinterpret_cast<f32x4 *>(w + lay.gt1);
+    bool forked;
     if ((rc = pair_sort_once(idx0, idx1, B, K, N, w + lay.sort[0], reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0],
-                             s)) != SFT_OK)
+                             &forked, s)) != SFT_OK)
       return rc;
     SideJoinGuard side_join(s);
+    if (!forked) side_join.release();
     if ((rc = launch_bias_partial(grad0, B, L, lay.nparts, partial, gt, true, s, grad1, gt1)) != SFT_OK) return rc;
     side_join.release();
-    if ((rc = join_side(s)) != SFT_OK) return rc;
+    if (forked && (rc = join_side(s)) != SFT_OK) return rc;
     {
       ProfScope prof(kProfBwdTiled, s);
       if ((rc = launch_pair_gather(ss[0].sb, ss[0].pos, N, gt, gt1, B, K, map, dst, bf, s)) != SFT_OK) return rc;
@@ -2131,11 +2149,13 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   e.partial = reinterpret_cast<f32x4 *>(w + lay.partial);
   e.P = L - L1;
   SortedSlots ss[2];  // sorted on the side stream while the epilogue runs
+  bool forked = true;
   int rc = lay.one_launch ? pair_sort_once(idx0, idx1, B, K, N, w + lay.sort[0],
-                                           reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], s)
+                                           reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], &forked, s)
                           : pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s);
   if (rc != SFT_OK) return rc;
   SideJoinGuard side_join(s);  // until the side stream's marks are waited for
+  if (!forked) side_join.release();
   {
     ProfScope prof(kProfBwdEpilogue, s);
     hipLaunchKernelGGL(bwd_epilogue_kernel, dim3((unsigned)lay.nparts), dim3(kBlock), 0, s, e, map, B,
@@ -2147,7 +2167,7 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
                      reinterpret_cast<f32x4 *>(db), 1};
   if (lay.one_launch) {
     side_join.release();
-    if ((rc = join_side(s)) != SFT_OK) return rc;
+    if (forked && (rc = join_side(s)) != SFT_OK) return rc;
     {
       ProfScope prof(kProfBwdTiled, s);
       if ((rc = launch_pair_gather(ss[0].sb, ss[0].pos, N, gt0, gt1, B, K, map, dst, bf, s)) != SFT_OK)
