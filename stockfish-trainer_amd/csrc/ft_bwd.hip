@@ -609,8 +609,7 @@ __device__ __forceinline__ void bwd_list_sum(const P *list, int n, int nmin, int
 // issued whole before anything waits on it: (1) the segment bounds; (2) the
 // positions (8 loads per thread in flight) together with, for kDstOutPlus, the
 // rows the sums add onto -- thread i loads chunk i % 8 of feature i / 8 into
-// LDS.  Meanwhile wave 0 ranks the 32 features by segment length with
-// cross-lane reads.  One barrier, then each lane group sums one feature,
+// LDS.  Meanwhile every wave ranks the 32 features by segment length.  One barrier, then each lane group sums one feature,
 // starting from the sum the previous position chunk left, which the lane
 // loads itself beside its first row loads.  (Staging one position per thread
 // per round trip, reading the segment bounds again after the ranking barrier
@@ -695,9 +694,11 @@ struct TiledArgs {
   int src_mode, dst_mode, ntiles, ngroups;
   const int32_t *long_list;
   const int *long_count;
-  int nlong;
+  int nlong, long_period;
   // workgroups from gblocks on reduce the bias partials instead (bias_final_block)
   int64_t gblocks;
+  uint32_t nl_items;           // workgroups of the long-segment slots, first in the grid
+  TileSched slots, features;  // (tile, slot) and (tile group, feature block) of a workgroup
   const f32x4 *bpart;
   int bparts;
   int64_t bcols;
@@ -705,7 +706,6 @@ struct TiledArgs {
   int boverwrite;
   int tile_group;  // tiles per workgroup (1: the single-tile kernel)
   const f32x4 *gt1;  // bwd_pair_gather_kernel: perspective 1's grad tiles
-  int long_period;
 };
 
 // Long-segment slot it.chunk of tile it.tile (whole workgroup).
@@ -720,24 +720,26 @@ __device__ __forceinline__ void tiled_long_item(const TiledArgs &a, TileItem it,
   }
 }
 
-// Copies cnt4 16-byte pieces of a position stream to LDS, 16-bit offsets (P16)
-// widened to ints, four loads per thread in flight.
+// A position stream's 16-byte pieces on their way to LDS: at most kBwdPosLds
+// entries, so one batch of loads, issued before the ranking and stored after it.
 template <bool P16>
-__device__ __forceinline__ void stage_positions(const void *__restrict__ from, int cnt4, int *to) {
-  constexpr int U = 4;
-  const int tid = threadIdx.x;
-  const i32x4 *src = reinterpret_cast<const i32x4 *>(from);
-  i32x4 *dst4 = reinterpret_cast<i32x4 *>(to);
-  for (int b0 = 0; b0 < cnt4; b0 += U * kBlock) {
-    i32x4 v[U];
+struct PositionPieces {
+  static constexpr int U = kBwdPosLds / (P16 ? 8 : 4) / kBlock;
+  i32x4 v[U];
+  __device__ __forceinline__ void load(const void *__restrict__ from, int cnt4) {
+    const i32x4 *src = reinterpret_cast<const i32x4 *>(from);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = b0 + u * kBlock + tid;
+      const int i = u * kBlock + (int)threadIdx.x;
       v[u] = i < cnt4 ? SFT_STREAM_LOAD(src + i) : i32x4{0, 0, 0, 0};
     }
+  }
+  // 16-bit offsets (P16) widened to ints
+  __device__ __forceinline__ void store(int cnt4, int *to) const {
+    i32x4 *dst4 = reinterpret_cast<i32x4 *>(to);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int i = b0 + u * kBlock + tid;
+      const int i = u * kBlock + (int)threadIdx.x;
       if (i >= cnt4) continue;
       if (P16) {
         const uint32_t w0 = (uint32_t)v[u][0], w1 = (uint32_t)v[u][1], w2 = (uint32_t)v[u][2], w3 = (uint32_t)v[u][3];
@@ -748,25 +750,34 @@ __device__ __forceinline__ void stage_positions(const void *__restrict__ from, i
       }
     }
   }
-}
+};
 
-// A wave runs as long as its longest segment: wave 0 ranks the block's features
-// (lane l's length is len) by length, ties by index, into s_perm, so that each
-// wave gets 8 consecutive ranks.
-__device__ __forceinline__ void rank_features(int len, int lane, int *s_perm) {
-  int rank = 0;
-  for (int j = 0; j < kBwdFeat; ++j) {
-    const int o = __builtin_amdgcn_readlane(len, j);
-    rank += (o > len || (o == len && j < lane)) ? 1 : 0;
+// A wave runs as long as its longest segment, so the block's 32 features are
+// ranked by length (lane l's is len < 2^9; ties by index) and each wave takes 8
+// consecutive ranks: returns the feature of rank `lane` (lanes 0-31).  Compared
+// bit by bit, all features at once -- nine ballots: the lanes that agreed so far
+// and have the bit this lane lacks are longer -- which is cheap enough for every
+// wave to rank by itself while the positions load, with nothing to wait for
+// behind the barrier (by 32 cross-lane reads in wave 0, the others waiting: a
+// backward of 65 536 positions, L = 1048 517 -> 499 us, encoded ones 452 -> 434).
+__device__ __forceinline__ int ranked_feature(int len, int lane) {
+  static_assert(kBwdFeat == 32, "one bit per feature");
+  uint32_t same = ~0u, longer = 0u;
+#pragma unroll
+  for (int j = 8; j >= 0; --j) {
+    const bool bit = (len >> j) & 1;
+    const uint32_t with = (uint32_t)ballot(bit);
+    longer |= bit ? 0u : same & with;
+    same &= bit ? with : ~with;
   }
-  if (lane < kBwdFeat) s_perm[rank] = lane;
+  const int rank = __popc(longer) + __popc(same & ((1u << (lane & 31)) - 1u));
+  return __builtin_amdgcn_ds_permute(4 * (lane < kBwdFeat ? rank : lane), lane);
 }
 
 // Feature block it.chunk of tile it.tile, or (MT) of the tile_group tiles from
 // tile_group * it.tile (whole workgroup; one barrier inside).
 template <bool NT, bool P16, bool MT>
-__device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem it, char *gsm, int *s_seg,
-                                                   int *s_perm) {
+__device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem it, char *gsm) {
   constexpr int TCH = kBwdTileCh;
   const int32_t *__restrict__ seg = a.seg;
   const int32_t *__restrict__ sorted_pos = a.sorted_pos;
@@ -786,18 +797,17 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
   const int64_t fb = (int64_t)it.chunk * kBwdFeat;
   const int nf = (int)(N - fb < kBwdFeat ? N - fb : kBwdFeat);  // features of this block, >= 1
 
-  // load round 1: segment bounds -- the range (uniform), this thread's feature for
-  // the start rows, and one feature per lane of wave 0 for the ranking
+  // load round 1: segment bounds -- the range (uniform), one feature per lane for
+  // the ranking and, with plus rows, this thread's feature for those
   const int r0 = seg[fb], r1 = seg[fb + nf];
-  const int64_t fs = fb + tid / TCH;  // start-row feature of this thread
+  const int64_t fs = fb + tid / TCH;  // plus-row feature of this thread
   const int cs = tid % TCH;
   int as = 0, es = 0;
-  if (fs < N) {
+  if (!MT && lay.plus >= 0 && fs < N) {
     as = seg[fs];
     es = seg[fs + 1];
   }
-  int la = 0;
-  if (wave == 0) la = seg[fb + (lane < nf ? lane : nf)];
+  const int la = seg[fb + (lane < nf ? lane : nf)];
 
   // load round 2: positions, start rows, plus rows.  The range is copied in
   // 16-byte pieces from r0 rounded down to a piece boundary (the position
@@ -808,9 +818,9 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
   const int ra = r0 & ~(PER - 1);
   const int cnt4 = (r1 - ra + PER - 1) / PER;           // 16-byte pieces
   const bool staged = cnt4 * PER <= kBwdPosLds;         // block-uniform
+  PositionPieces<P16> pieces;
   if (staged)
-    stage_positions<P16>(P16 ? static_cast<const void *>(pos16 + ra) : static_cast<const void *>(sorted_pos + ra), cnt4,
-                         spos);
+    pieces.load(P16 ? static_cast<const void *>(pos16 + ra) : static_cast<const void *>(sorted_pos + ra), cnt4);
   if (!MT && lay.plus >= 0) {
     const int colm = tile_col(map, it.tile, cs);
     f32x4 vp = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -820,18 +830,15 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
     }
     reinterpret_cast<f32x4 *>(gsm + lay.plus)[tid] = vp;
   }
-  if (wave == 0) {
-    const int le = __shfl_down(la, 1);
-    const bool live = lane < nf;
-    rank_features((live && !long_segment(la, le, a.long_period)) ? le - la : 0, lane, s_perm);  // long segments as 0
-    if (lane <= kBwdFeat) s_seg[lane] = la;
-  }
+  const int g = lane / TCH, t = lane % TCH;
+  const int le = __shfl_down(la, 1);
+  const int ranked = ranked_feature(lane < nf && !long_segment(la, le, a.long_period) ? le - la : 0, lane);  // long as 0
+  const int p = __shfl(ranked, wave * (kWave / TCH) + g);
+  const int64_t f = fb + p;
+  const int s0 = __shfl(la, p), s1 = __shfl(la, p + 1);
+  if (staged) pieces.store(cnt4, spos);
   __syncthreads();
 
-  const int g = lane / TCH, t = lane % TCH;
-  const int p = s_perm[wave * (kWave / TCH) + g];
-  const int64_t f = fb + p;
-  const int s0 = s_seg[p], s1 = s_seg[p + 1];
   const bool live = p < nf;
   const bool is_long = live && long_segment(s0, s1, a.long_period);  // summed by the long-segment slots
   const int n = (live && !is_long) ? s1 - s0 : 0;
@@ -892,21 +899,18 @@ __device__ __forceinline__ void tiled_feature_item(const TiledArgs &a, TileItem 
 template <bool NT, bool P16, bool MT>
 __global__ __launch_bounds__(kBlock) void bwd_tiled_gather_kernel(TiledArgs a) {
   extern __shared__ __align__(16) char gsm[];
-  __shared__ int s_seg[kBwdFeat + 1], s_perm[kBwdFeat];
   if ((int64_t)blockIdx.x >= a.gblocks) {  // whole block: uniform
     bias_final_block<f32x4>((int64_t)blockIdx.x - a.gblocks, a.bpart, a.bparts, a.bcols, a.db, a.boverwrite);
     return;
   }
-  const int64_t nl_items = tile_sched_items_per_xcd(a.ntiles, a.nlong) * kXcds;
-  const bool long_item = (int64_t)blockIdx.x < nl_items;  // whole block: uniform
-  const int nt = MT && !long_item ? (a.ntiles + a.tile_group - 1) / a.tile_group : a.ntiles;
-  const TileItem it = long_item ? tile_sched_item(blockIdx.x, nt, a.nlong)
-                                : tile_sched_item(blockIdx.x - nl_items, nt, a.ngroups);
-  if (it.tile >= nt) return;  // whole block: uniform
-  if (long_item)
-    tiled_long_item(a, it, gsm);
-  else
-    tiled_feature_item<NT, P16, MT>(a, it, gsm, s_seg, s_perm);
+  if (blockIdx.x < a.nl_items) {  // whole block: uniform
+    const TileItem it = a.slots.item(blockIdx.x);
+    if (it.tile < a.ntiles) tiled_long_item(a, it, gsm);
+    return;
+  }
+  const TileItem it = a.features.item(blockIdx.x - a.nl_items);
+  if (it.tile >= a.features.ntiles) return;  // whole block: uniform
+  tiled_feature_item<NT, P16, MT>(a, it, gsm);
 }
 
 
@@ -924,15 +928,13 @@ template <bool NT>
 __global__ __launch_bounds__(kBlock) void bwd_pair_gather_kernel(TiledArgs a) {
   constexpr int TCH = kBwdTileCh;
   extern __shared__ __align__(16) char gsm[];
-  __shared__ int s_seg[2][kBwdFeat + 1], s_perm[kBwdFeat];
   if ((int64_t)blockIdx.x >= a.gblocks) {  // whole block: uniform
     bias_final_block<f32x4>((int64_t)blockIdx.x - a.gblocks, a.bpart, a.bparts, a.bcols, a.db, a.boverwrite);
     return;
   }
   const int64_t N = a.N;
-  const int64_t nl_items = tile_sched_items_per_xcd(a.ntiles, a.nlong) * kXcds;
-  if ((int64_t)blockIdx.x < nl_items) {  // a long-segment slot: features long in either perspective
-    const TileItem it = tile_sched_item(blockIdx.x, a.ntiles, a.nlong);
+  if (blockIdx.x < a.nl_items) {  // a long-segment slot: features long in either perspective
+    const TileItem it = a.slots.item(blockIdx.x);
     if (it.tile >= a.ntiles) return;
     const int c0 = a.long_count[0], cnt = c0 + a.long_count[1];
     f32x4 *buf = reinterpret_cast<f32x4 *>(gsm);
@@ -951,46 +953,47 @@ __global__ __launch_bounds__(kBlock) void bwd_pair_gather_kernel(TiledArgs a) {
     }
     return;
   }
-  const int ngrp = (a.ntiles + a.tile_group - 1) / a.tile_group;
-  const TileItem it = tile_sched_item(blockIdx.x - nl_items, ngrp, a.ngroups);
-  if (it.tile >= ngrp) return;  // whole block: uniform
+  const TileItem it = a.features.item(blockIdx.x - a.nl_items);
+  if (it.tile >= a.features.ntiles) return;  // whole block: uniform
   const int tid = threadIdx.x, wave = uniform(tid / kWave), lane = tid % kWave;
   const int64_t fb = (int64_t)it.chunk * kBwdFeat;
   const int nf = (int)(N - fb < kBwdFeat ? N - fb : kBwdFeat);
   int *spos = reinterpret_cast<int *>(gsm);
   // as in tiled_feature_item: the ranges' bounds, then their positions
-  int r0[2], r1[2], la[2] = {0, 0};
+  int r0[2], r1[2], la[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     r0[p] = a.seg[p * N + fb];
     r1[p] = a.seg[p * N + fb + nf];
-    if (wave == 0) la[p] = a.seg[p * N + fb + (lane < nf ? lane : nf)];
+    la[p] = a.seg[p * N + fb + (lane < nf ? lane : nf)];
   }
   constexpr int PER = 8;
   const int ra0 = r0[0] & ~(PER - 1), ra1 = r0[1] & ~(PER - 1);
   const int cnt0 = (r1[0] - ra0 + PER - 1) / PER, cnt1 = (r1[1] - ra1 + PER - 1) / PER;
   const bool staged = (cnt0 + cnt1) * PER <= kBwdPosLds;  // block-uniform
+  PositionPieces<true> pieces[2];
   if (staged) {
-    stage_positions<true>(a.pos16 + ra0, cnt0, spos);
-    stage_positions<true>(a.pos16 + ra1, cnt1, spos + cnt0 * PER);
+    pieces[0].load(a.pos16 + ra0, cnt0);
+    pieces[1].load(a.pos16 + ra1, cnt1);
   }
-  if (wave == 0) {
-    int len = 0;
-    bool any_long = false;
+  int len = 0;
+  bool any_long = false;
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int le = __shfl_down(la[p], 1);
-      any_long = any_long || long_segment(la[p], le, a.long_period);
-      len += le - la[p];
-      if (lane <= kBwdFeat) s_seg[p][lane] = la[p];
-    }
-    rank_features(lane < nf && !any_long ? len : 0, lane, s_perm);
+  for (int p = 0; p < 2; ++p) {
+    const int le = __shfl_down(la[p], 1);
+    any_long = any_long || long_segment(la[p], le, a.long_period);
+    len += le - la[p];
+  }
+  const int g = lane / TCH, t = lane % TCH;
+  const int ranked = ranked_feature(lane < nf && !any_long ? len : 0, lane);
+  const int f32 = __shfl(ranked, wave * (kWave / TCH) + g);
+  const int s0 = __shfl(la[0], f32), s1 = __shfl(la[0], f32 + 1), u0 = __shfl(la[1], f32), u1 = __shfl(la[1], f32 + 1);
+  if (staged) {
+    pieces[0].store(cnt0, spos);
+    pieces[1].store(cnt1, spos + cnt0 * PER);
   }
   __syncthreads();
 
-  const int g = lane / TCH, t = lane % TCH;
-  const int f32 = s_perm[wave * (kWave / TCH) + g];
-  const int s0 = s_seg[0][f32], s1 = s_seg[0][f32 + 1], u0 = s_seg[1][f32], u1 = s_seg[1][f32 + 1];
   const bool live = f32 < nf && !long_segment(s0, s1, a.long_period) && !long_segment(u0, u1, a.long_period);
   const int n0 = live ? s1 - s0 : 0, n1 = live ? u1 - u0 : 0;
   int min0, max0, min1, max1;
@@ -1078,15 +1081,16 @@ int launch_tiled_gather(bool nt, const int32_t *seg, const int32_t *pos, const u
                         const BiasFinal *bias = nullptr) {
   const bool one_chunk = src_mode == kSrcZero && dst_mode != kDstTmp;
   const int tg = one_chunk && pos16 != nullptr ? gather_tile_group(B, ntiles, ngroups) : 1;
-  const int64_t items = tile_sched_items_per_xcd(ntiles, nlong) +
-                        tile_sched_items_per_xcd((int)ceil_div(ntiles, tg), ngroups);
+  const TileSched slots(ntiles, nlong), features((int)ceil_div(ntiles, tg), ngroups);
+  const int64_t nl_items = tile_sched_items_per_xcd(ntiles, nlong) * kXcds;
+  const int64_t gblocks = nl_items + tile_sched_items_per_xcd(features.ntiles, ngroups) * kXcds;
   const size_t lds = (size_t)gather_lds(tg > 1 ? kDstOut : dst_mode).bytes;
   if ((uintptr_t)pos % 16 != 0 || (uintptr_t)pos16 % 16 != 0)  // 256-byte / 16-byte aligned workspace regions
     return fail(SFT_EINVAL, "tiled feature gather: sorted positions not 16-byte aligned");
-  const int64_t gblocks = items * kXcds;
   const TiledArgs a{seg, pos, pos16, (int)chunk_base, N, gt, B, map, dst, tmp, src_mode, dst_mode, ntiles, ngroups,
-                    long_list, long_count, nlong, gblocks, bias ? bias->partial : nullptr, bias ? bias->nparts : 0,
-                    bias ? bias->cols : 0, bias ? bias->db : nullptr, bias ? bias->overwrite : 0, tg, nullptr, long_period};
+                    long_list, long_count, nlong, long_period, gblocks, (uint32_t)nl_items, slots, features,
+                    bias ? bias->partial : nullptr, bias ? bias->nparts : 0,
+                    bias ? bias->cols : 0, bias ? bias->db : nullptr, bias ? bias->overwrite : 0, tg, nullptr};
   const bool p16 = pos16 != nullptr;
   const dim3 grid((unsigned)(gblocks + (bias ? bias_final_blocks(bias->cols) : 0)));
   if (tg > 1)
@@ -1106,12 +1110,13 @@ int launch_pair_gather(const SegBufs &sb, const int32_t *pos, int64_t N, const f
   const int ngroups = (int)ceil_div(N, kBwdFeat);
   const int tg = gather_tile_group(2 * B, ntiles, ngroups);
   const int period = long_period(B, K, N), nlong = long_slots(2 * B * K, period);
-  const int64_t gblocks =
-      (tile_sched_items_per_xcd(ntiles, nlong) + tile_sched_items_per_xcd((int)ceil_div(ntiles, tg), ngroups)) * kXcds;
+  const TileSched slots(ntiles, nlong), features((int)ceil_div(ntiles, tg), ngroups);
+  const int64_t nl_items = tile_sched_items_per_xcd(ntiles, nlong) * kXcds;
+  const int64_t gblocks = nl_items + tile_sched_items_per_xcd(features.ntiles, ngroups) * kXcds;
   if ((uintptr_t)sb.pos16 % 16 != 0) return fail(SFT_EINVAL, "pair feature gather: sorted positions not 16-byte aligned");
   const TiledArgs a{sb.seg, pos, sb.pos16, 0, N, gt0, B, map, dst, nullptr, kSrcZero, kDstOut, ntiles, ngroups,
-                    sb.list, sb.count, nlong, gblocks, bias.partial, bias.nparts, bias.cols, bias.db, bias.overwrite,
-                    tg, gt1, period};
+                    sb.list, sb.count, nlong, period, gblocks, (uint32_t)nl_items, slots, features, bias.partial, bias.nparts, bias.cols, bias.db,
+                    bias.overwrite, tg, gt1};
   const dim3 grid((unsigned)(gblocks + bias_final_blocks(bias.cols)));
   const size_t lds = (size_t)gather_lds(kDstOut).bytes;
   hipLaunchKernelGGL((B * kBwdTileCh * 16 >= kNtStoreTileBytes ? bwd_pair_gather_kernel<true> : bwd_pair_gather_kernel<false>),

@@ -797,13 +797,24 @@ __global__ __launch_bounds__(kWideBlock) void rank_lists_wide_kernel(RankArgs a,
 // every block, and so on (the last block may hold fewer chunks) -- so a tile
 // pass starts with its longest items and ends with its shortest.
 constexpr int kChunksPerSortBlock = kRankSortBlock / kRanksPerBlock;  // 8
-__device__ __forceinline__ int64_t rank_chunk(int64_t c, int64_t nchunks) {
-  const int64_t nb = (nchunks + kChunksPerSortBlock - 1) / kChunksPerSortBlock;  // sort blocks
-  const int64_t last = nchunks - (nb - 1) * kChunksPerSortBlock;                 // chunks of the last block
-  if (c < last * nb) return (c % nb) * kChunksPerSortBlock + c / nb;
-  const int64_t c2 = c - last * nb;
-  return (c2 % (nb - 1)) * kChunksPerSortBlock + last + c2 / (nb - 1);
-}
+struct RankChunks {
+  uint32_t nb, last;      // sort blocks; chunks of the last block
+  FastDiv by_nb, by_nb1;  // / nb, / (nb - 1)
+  RankChunks() = default;
+  explicit RankChunks(int64_t nchunks)
+      : nb((uint32_t)ceil_div(nchunks, (int64_t)kChunksPerSortBlock)),
+        last((uint32_t)(nchunks - (int64_t)(nb - 1) * kChunksPerSortBlock)),
+        by_nb(nb),
+        by_nb1(nb > 1 ? nb - 1 : 1) {}
+  __device__ __forceinline__ uint32_t operator()(uint32_t c) const {
+    if (c < last * nb) {
+      const uint32_t q = by_nb(c);
+      return (c - q * nb) * kChunksPerSortBlock + q;
+    }
+    const uint32_t c2 = c - last * nb, q = by_nb1(c2);
+    return (c2 - q * (nb - 1)) * kChunksPerSortBlock + last + q;
+  }
+};
 
 // The whole lists of ranks r0 .. r0 + 7 (a wave's 8, padded to kpad) into the
 // wave's LDS lists, 16-bit entries widened to ints.
@@ -840,12 +851,13 @@ __global__ __launch_bounds__(kBlock) void fwd_tiled_kernel(RankLists R0, RankLis
                                                            const f32x4 *__restrict__ Wt, ColMap map,
                                                            const f32x4 *__restrict__ bias, f32x4 *__restrict__ out0,
                                                            f32x4 *__restrict__ out1, FwdEpilogue epi, int kpad,
-                                                           int ntiles, int nchunks, int nchunks_p, int part,
+                                                           TileSched sched, RankChunks chunk_of, int nchunks_p, int part,
                                                            int nparts, f32x4 *__restrict__ carry0,
                                                            f32x4 *__restrict__ carry1, int64_t B) {
   constexpr int PPW = kWave / kTileCh;  // 8 ranks per wave
   extern __shared__ int smem[];         // 8 lists of kpad entries per wave
-  TileItem it = tile_sched_item(blockIdx.x, ntiles, nchunks);
+  const int ntiles = sched.ntiles;
+  TileItem it = sched.item(blockIdx.x);
   if (it.tile >= ntiles) return;  // whole block: uniform
   const bool second = it.chunk >= nchunks_p;
   if (second) it.chunk -= nchunks_p;
@@ -861,7 +873,7 @@ __global__ __launch_bounds__(kBlock) void fwd_tiled_kernel(RankLists R0, RankLis
   const char *tbase = reinterpret_cast<const char *>(Wt + (int64_t)it.tile * tile_rows(N) * kTileCh);
   const uint32_t lane_off = (uint32_t)t * (uint32_t)sizeof(f32x4);
 
-  const int64_t r0 = rank_chunk(it.chunk, nchunks_p) * kRanksPerBlock + wave * PPW;  // the wave's first rank
+  const int64_t r0 = (int64_t)chunk_of(it.chunk) * kRanksPerBlock + wave * PPW;  // the wave's first rank
   int *list = smem + wave * PPW * kpad;
   const int32_t *__restrict__ rp = R.pos + r0;
   int pos = rp[0];
@@ -1102,13 +1114,13 @@ __global__ __launch_bounds__(kBlock) void fwd_i16_tiled_kernel(const int32_t *__
                                                                i16x8 *__restrict__ out0, i16x8 *__restrict__ out1,
                                                                int32_t *__restrict__ psqt_out0,
                                                                int32_t *__restrict__ psqt_out1, int clip_lo,
-                                                               int clip_hi, int wrap16, int kpad, int ntiles,
-                                                               int nchunks, int nchunks_p) {
+                                                               int clip_hi, int wrap16, int kpad, TileSched sched,
+                                                               int nchunks_p) {
   constexpr int PPW = kWave / kTileCh;
   static_assert(PPW <= kCompactRows, "compact_rows takes at most kCompactRows rows");
   extern __shared__ int smem[];
-  TileItem it = tile_sched_item(blockIdx.x, ntiles, nchunks);
-  if (it.tile >= ntiles) return;
+  TileItem it = sched.item(blockIdx.x);
+  if (it.tile >= sched.ntiles) return;
   const bool second = it.chunk >= nchunks_p;  // block-uniform
   if (second) it.chunk -= nchunks_p;
   const int32_t *__restrict__ idx = second ? idx1 : idx0;
@@ -1168,12 +1180,12 @@ __global__ __launch_bounds__(kBlock) void fwd_i16_ranked_kernel(RankLists R0, Ra
                                                                 i16x8 *__restrict__ out0, i16x8 *__restrict__ out1,
                                                                 int32_t *__restrict__ psqt_out0,
                                                                 int32_t *__restrict__ psqt_out1, int clip_lo,
-                                                                int clip_hi, int wrap16, int kpad, int ntiles,
-                                                                int nchunks, int nchunks_p) {
+                                                                int clip_hi, int wrap16, int kpad, TileSched sched,
+                                                                RankChunks chunk_of, int nchunks_p) {
   constexpr int PPW = kWave / kTileCh;  // 8 ranks per wave
   extern __shared__ int smem[];         // 8 lists of kpad entries per wave
-  TileItem it = tile_sched_item(blockIdx.x, ntiles, nchunks);
-  if (it.tile >= ntiles) return;  // whole block: uniform
+  TileItem it = sched.item(blockIdx.x);
+  if (it.tile >= sched.ntiles) return;  // whole block: uniform
   const bool second = it.chunk >= nchunks_p;  // block-uniform
   if (second) it.chunk -= nchunks_p;
   const RankLists R = second ? R1 : R0;
@@ -1191,7 +1203,7 @@ __global__ __launch_bounds__(kBlock) void fwd_i16_ranked_kernel(RankLists R0, Ra
   const uint32_t lane_off = (uint32_t)t * (uint32_t)sizeof(i16x8);
   const i32x8 b8 = colok ? Q16<i16x8>::widen(bias[col]) : (i32x8)0;
 
-  const int64_t r0 = rank_chunk(it.chunk, nchunks_p) * kRanksPerBlock + wave * PPW;  // the wave's first rank
+  const int64_t r0 = (int64_t)chunk_of(it.chunk) * kRanksPerBlock + wave * PPW;  // the wave's first rank
   int *list = smem + wave * PPW * kpad;
   const int32_t *__restrict__ rp = R.pos + r0;
   const int32_t *__restrict__ rc = R.count + r0;
@@ -1618,7 +1630,8 @@ int fwd_f32_tiled(const int32_t *idx, int64_t B, int K, const float *W, int64_t 
     hipLaunchKernelGGL((nparts > 1 ? fwd_tiled_kernel<false, true> : fwd_tiled_kernel<false, false>),
                        dim3((unsigned)blocks), dim3(kBlock), lds, s, R, R, (int)N, wt,
                        plain_map((int)cols4), reinterpret_cast<const f32x4 *>(bias), reinterpret_cast<f32x4 *>(out),
-                       reinterpret_cast<f32x4 *>(out), FwdEpilogue{}, kpad, ntiles, nchunks, nchunks, part, nparts,
+                       reinterpret_cast<f32x4 *>(out), FwdEpilogue{}, kpad, TileSched(ntiles, nchunks),
+                       RankChunks(nchunks), nchunks, part, nparts,
                        carry, carry, B);
     if ((rc = check_launch("sft_ft_fwd_f32_ex (tiled gather)")) != SFT_OK) return rc;
   }
@@ -1670,18 +1683,20 @@ static int pair_gather(const int32_t *idx0, const int32_t *idx1, int64_t B, int 
   if ((rc = build_rank_lists(idx0, idx1, 2, B, K, (int)N, R0, R1, nparts, s, who)) != SFT_OK) return rc;
   const int nchunks_p = (int)(rank_pad(B) / kRanksPerBlock);
   const int64_t blocks = tile_sched_items_per_xcd(ntiles, 2 * nchunks_p) * kXcds;
+  const TileSched sched(ntiles, 2 * nchunks_p);
+  const RankChunks chunk_of(nchunks_p);
   for (int part = 0; part < nparts; ++part) {
     ProfScope prof(kProfFwdTiled, s);
     if (epi.l0 != nullptr)
       hipLaunchKernelGGL((nparts > 1 ? fwd_tiled_kernel<true, true> : fwd_tiled_kernel<true, false>),
                          dim3((unsigned)blocks), dim3(kBlock), lds, s, R0, R1, (int)N, wt,
                          map, reinterpret_cast<const f32x4 *>(bias), (f32x4 *)nullptr, (f32x4 *)nullptr, epi, kpad,
-                         ntiles, 2 * nchunks_p, nchunks_p, part, nparts, carry0, carry1, B);
+                         sched, chunk_of, nchunks_p, part, nparts, carry0, carry1, B);
     else
       hipLaunchKernelGGL((nparts > 1 ? fwd_tiled_kernel<false, true> : fwd_tiled_kernel<false, false>),
                          dim3((unsigned)blocks), dim3(kBlock), lds, s, R0, R1, (int)N, wt,
                          map, reinterpret_cast<const f32x4 *>(bias), reinterpret_cast<f32x4 *>(out0),
-                         reinterpret_cast<f32x4 *>(out1), epi, kpad, ntiles, 2 * nchunks_p, nchunks_p, part, nparts,
+                         reinterpret_cast<f32x4 *>(out1), epi, kpad, sched, chunk_of, nchunks_p, part, nparts,
                          carry0, carry1, B);
     if ((rc = check_launch(who)) != SFT_OK) return rc;
   }
@@ -1771,8 +1786,8 @@ int fwd_i16_packed(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, c
                        persp == 2 ? idx1 : idx0, B, K, (int)N, static_cast<const i16x8 *>(packed), (int64_t)cols8,
                        pch, reinterpret_cast<const i16x8 *>(bias), P, reinterpret_cast<i16x8 *>(out0),
                        reinterpret_cast<i16x8 *>(persp == 2 ? out1 : out0), psqt_out0,
-                       persp == 2 ? psqt_out1 : psqt_out0, lo, hi, wrap16, kpad, ntiles, persp * nchunks_p,
-                       nchunks_p);
+                       persp == 2 ? psqt_out1 : psqt_out0, lo, hi, wrap16, kpad,
+                       TileSched(ntiles, persp * nchunks_p), nchunks_p);
   }
   return check_launch((std::string(who) + " (tiled gather)").c_str());
 }
@@ -1809,8 +1824,8 @@ int fwd_i16_packed_ranked(const int32_t *idx0, const int32_t *idx1, int64_t B, i
     hipLaunchKernelGGL(fwd_i16_ranked_kernel, dim3((unsigned)blocks), dim3(kBlock), lds, s, R0, R1, (int)N,
                        static_cast<const i16x8 *>(packed), (int64_t)cols8, pch, reinterpret_cast<const i16x8 *>(bias),
                        P, reinterpret_cast<i16x8 *>(out0), reinterpret_cast<i16x8 *>(persp == 2 ? out1 : out0),
-                       psqt_out0, persp == 2 ? psqt_out1 : psqt_out0, lo, hi, wrap16, kpad, ntiles,
-                       persp * nchunks_p, nchunks_p);
+                       psqt_out0, persp == 2 ? psqt_out1 : psqt_out0, lo, hi, wrap16, kpad,
+                       TileSched(ntiles, persp * nchunks_p), RankChunks(nchunks_p), nchunks_p);
   }
   return check_launch((std::string(who) + " (ranked gather)").c_str());
 }

@@ -75,29 +75,50 @@ SFT_HD inline int64_t tile_sched_items_per_xcd(int ntiles, int nchunks) {
   const int full = ntiles / kXcds, rem = ntiles % kXcds;
   return (int64_t)full * nchunks + (int64_t)rem * ((nchunks + kXcds - 1) / kXcds);
 }
-SFT_HD inline TileItem tile_sched_item(int64_t bid, int ntiles, int nchunks) {
-  const int xcd = (int)(bid % kXcds);
-  const int64_t j = bid / kXcds;
-  const int full = ntiles / kXcds, rem = ntiles % kXcds;
-  const int64_t fj = (int64_t)full * nchunks;
-  if (j < fj) return TileItem{xcd + kXcds * (int)(j / nchunks), (int)(j % nchunks)};
-  if (rem == 0) return TileItem{ntiles, 0};  // no work
-  const int64_t rounds = (nchunks + kXcds - 1) / kXcds;  // chunks per strand, the last round partial
-  const int s0 = xcd * rem;                              // first strand of this XCD
-  const int ta = s0 / kXcds;                             // its first leftover tile
-  const int na = ((ta + 1) * kXcds < s0 + rem ? (ta + 1) * kXcds : s0 + rem) - s0;  // strands of tile ta
-  int64_t i = j - fj;
-  int t = ta, s = s0 % kXcds, n = na;
-  if (i >= rounds * na) {  // strands 0 .. rem - na - 1 of the next leftover tile
-    i -= rounds * na;
-    t = ta + 1;
-    s = 0;
-    n = rem - na;
-    if (n <= 0) return TileItem{ntiles, 0};  // no work
+// The item of a workgroup, in 32-bit arithmetic with the chunk count's magic
+// divisor made at launch: every workgroup starts with it, and 64-bit divisions
+// there cost a tiled gather's workgroup about a tenth of a microsecond each.
+struct TileSched {
+  int ntiles, nchunks;
+  FastDiv by_chunks;
+  TileSched() = default;
+  SFT_HD TileSched(int tiles, int chunks) : ntiles(tiles), nchunks(chunks), by_chunks((uint32_t)(chunks > 0 ? chunks : 1)) {}
+  // i / n for n <= 7, i < 2^29: i * ceil(2^32 / n) >> 32.
+  static SFT_HD uint32_t div_small(uint32_t i, uint32_t n) {
+    const uint32_t m = n == 2 ? 0x80000000u : n == 3 ? 0x55555556u : n == 4 ? 0x40000000u : n == 5 ? 0x33333334u
+                       : n == 6 ? 0x2aaaaaabu : 0x24924925u;
+    return n <= 1 ? i : mulhi32(i, m);
   }
-  const int64_t c = (i / n) * kXcds + s + i % n;
-  if (c >= nchunks) return TileItem{ntiles, 0};  // no work: past a strand's end
-  return TileItem{kXcds * full + t, (int)c};
+  SFT_HD TileItem item(uint32_t bid) const {
+    const uint32_t xcd = bid % kXcds, j = bid / kXcds;
+    const uint32_t full = (uint32_t)ntiles / kXcds, rem = (uint32_t)ntiles % kXcds;
+    const uint32_t fj = full * (uint32_t)nchunks;
+    if (j < fj) {
+      const uint32_t t = by_chunks(j);
+      return TileItem{(int)(xcd + kXcds * t), (int)(j - t * (uint32_t)nchunks)};
+    }
+    if (rem == 0) return TileItem{ntiles, 0};  // no work
+    const uint32_t rounds = ((uint32_t)nchunks + kXcds - 1) / kXcds;  // chunks per strand, the last round partial
+    const uint32_t s0 = xcd * rem;                                    // first strand of this XCD
+    const uint32_t ta = s0 / kXcds;                                   // its first leftover tile
+    const uint32_t na = ((ta + 1) * kXcds < s0 + rem ? (ta + 1) * kXcds : s0 + rem) - s0;  // strands of tile ta
+    uint32_t i = j - fj;
+    uint32_t t = ta, s = s0 % kXcds, n = na;
+    if (i >= rounds * na) {  // strands 0 .. rem - na - 1 of the next leftover tile
+      i -= rounds * na;
+      t = ta + 1;
+      s = 0;
+      n = rem - na;
+      if (n == 0) return TileItem{ntiles, 0};  // no work
+    }
+    const uint32_t r = div_small(i, n);
+    const uint32_t c = r * kXcds + s + (i - r * n);
+    if (c >= (uint32_t)nchunks) return TileItem{ntiles, 0};  // no work: past a strand's end
+    return TileItem{(int)(kXcds * full + t), (int)c};
+  }
+};
+SFT_HD inline TileItem tile_sched_item(int64_t bid, int ntiles, int nchunks) {
+  return TileSched(ntiles, nchunks).item((uint32_t)bid);
 }
 
 // ---- column maps of the 32-column tiles ----
