@@ -5,7 +5,7 @@
 // key's positions come out in ascending order; inactive slots are dropped by
 // the first pass.  RB-bit digits (8, or 9 when two 9-bit passes cover a key
 // that 8-bit digits would need three for), least significant first; each pass:
-//   upsweep:   per 2048-slot tile, a 2^RB-bin digit histogram;
+//   upsweep:   per tile of 1024 or 4096 slots, a 2^RB-bin digit histogram;
 //   scan:      per digit, an exclusive scan of its tile counts and the digit
 //              total; a digit's base is the scan of the totals (done in the
 //              downsweep), so (digit, tile) starts at base + its tile prefix;
@@ -23,20 +23,22 @@ namespace sft {
 
 namespace {
 
-// Slots per thread of a sort tile: 8 (2048-slot tiles) for up to kBigSort
-// slots, 16 above, where fewer tiles shrink the per-tile digit counts the
-// scans walk (10.5 M slots: 278 -> 226 us per sort).  Alone, a 2.1 M-slot sort
-// was faster with 8 (65 vs 72 us), but beside the kernels it shares the GPU
-// with the steps are faster with 16 at every batch: B = 65536, L = 1048 1.671
-// -> 1.666 ms, L = 136 0.378 -> 0.376 ms, B = 16384 0.575 -> 0.574 ms (A/B
-// builds, same box), so the threshold is 0.
-constexpr int kSortItems = 8;
-constexpr int kSortItemsBig = 16;
-#ifndef SFT_SORT_BIG_SLOTS
-#define SFT_SORT_BIG_SLOTS 0
-#endif
-constexpr int64_t kBigSort = SFT_SORT_BIG_SLOTS;
-constexpr int kSortTile = kBlock * kSortItems;  // the smaller tile: sizes the count buffer
+// Slots per thread of a sort tile: 4 (1024-slot tiles) up to kSmallSlots slots,
+// 16 above.  A small sort is a chain of latencies in a few workgroups: with
+// 4096-slot tiles 320 K slots filled 79 of them (downsweep 13.0 -> 7.8 us).  A
+// large one pays per tile, for its digit counts and the scans that walk them,
+// and shares the GPU: 2.1 M slots, both perspectives' steps with 4 / 8 / 16 per
+// thread, L = 136 387 / 369 / 366 us, L = 1048 1668 / 1645 / 1634 us.
+constexpr int64_t kSmallSlots = 1 << 19;
+constexpr int kSmallItems = 4, kBigItems = 16;
+inline bool sort_big(int64_t M) { return M > kSmallSlots; }
+inline int sort_tiles(int64_t M) {
+  return (int)ceil_div(std::max<int64_t>(M, 1), (int64_t)kBlock * (sort_big(M) ? kBigItems : kSmallItems));
+}
+// The count buffer's tiles: at least sort_tiles(M), and growing with M.
+inline int64_t max_sort_tiles(int64_t M) {
+  return std::max<int64_t>(sort_tiles(M), sort_tiles(std::min(M, kSmallSlots)));
+}
 constexpr int kMaxRadix = 1024;  // 10-bit digits (the bucket sort's first pass)
 #ifndef SFT_SORT_BUCKETS
 #define SFT_SORT_BUCKETS 1
@@ -272,10 +274,27 @@ __global__ __launch_bounds__(kBlock) void radix_downsweep(SlotKey sk, const unsi
   __shared__ unsigned dtot[R];
   __shared__ unsigned dbase[R];
   const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-  for (int d = tid; d < R; d += kBlock) {
+  constexpr int DPT = R / kBlock;  // digits per thread
+  unsigned tstart[DPT];            // this tile's start in each of the thread's digits
+#pragma unroll
+  for (int j = 0; j < DPT; ++j) {
+    const int d = tid + j * kBlock;
     dtot[d] = totals[d];
+    tstart[j] = offs[(int64_t)d * ntiles + blockIdx.x];
 #pragma unroll
     for (int w = 0; w < kWavesPerBlock; ++w) wrun[w][d] = 0;
+  }
+  const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)wave * PER_WAVE;
+  unsigned key[IT];
+  int val[IT];
+  unsigned rank[IT];
+  bool act[IT];
+  // loads from clamped indices, all issued before any is used (see the
+  // upsweep), the first pass's, which need no count, ahead of the digit bases
+  if (FIRST) {
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+      key[i] = sk.load(std::max<int64_t>(std::min<int64_t>(base + (int64_t)i * kWave + lane, M - 1), 0));
   }
   __syncthreads();
   if (wave == 1) wave_scan_digits<R>(dtot, dbase, lane);  // digit bases in the whole output
@@ -283,19 +302,14 @@ __global__ __launch_bounds__(kBlock) void radix_downsweep(SlotKey sk, const unsi
   // Elements read by this pass: all slots (first pass) or the active ones,
   // whose count is the sum of this pass's digit totals.
   const int64_t n_in = FIRST ? M : (int64_t)dbase[R - 1] + dtot[R - 1];
-  const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)wave * PER_WAVE;
-
-  unsigned key[IT];
-  int val[IT];
-  unsigned rank[IT];
-  bool act[IT];
-  // loads from clamped indices, all issued before any is used (see the upsweep)
   const int64_t last = n_in > 0 ? n_in - 1 : 0;
+  if (!FIRST) {
 #pragma unroll
-  for (int i = 0; i < IT; ++i) {
-    const int64_t ec = std::min<int64_t>(base + (int64_t)i * kWave + lane, last);
-    key[i] = FIRST ? sk.load(ec) : kin[ec];
-    if (!FIRST) val[i] = vin[ec];
+    for (int i = 0; i < IT; ++i) {
+      const int64_t ec = std::min<int64_t>(base + (int64_t)i * kWave + lane, last);
+      key[i] = kin[ec];
+      val[i] = vin[ec];
+    }
   }
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
@@ -342,12 +356,17 @@ __global__ __launch_bounds__(kBlock) void radix_downsweep(SlotKey sk, const unsi
     }
   }
   const int kept = (int)(dstart[R - 1] + dtot[R - 1]);  // active elements of the tile
+  // dbase: from the tile's order to the output (mod 2^32).  The tile's starts
+  // came with the first loads; read here, one per element, they made the store
+  // loop a chain of memory round trips (2.1 M slots 20.5 -> 16.5 us).
+#pragma unroll
+  for (int j = 0; j < DPT; ++j) dbase[tid + j * kBlock] += tstart[j] - dstart[tid + j * kBlock];
   __syncthreads();
 
   for (int j = tid; j < kept; j += kBlock) {
     const unsigned k = s_keys[j];
     const unsigned d = (k >> shift) & (R - 1);
-    const int64_t dst = (int64_t)dbase[d] + offs[(int64_t)d * ntiles + blockIdx.x] + (j - dstart[d]);
+    const unsigned dst = dbase[d] + (unsigned)j;
     kout[dst] = k;
     vout[dst] = s_vals[j];
   }
@@ -415,7 +434,6 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(
     int long_period, int b0) {
   constexpr int D = 1 << SB;
   constexpr int TILE = kBucketBlock * kBucketItems;
-  constexpr int PER_WAVE = TILE / kBucketWaves;
   __shared__ unsigned red[2][kBucketWaves];
   __shared__ unsigned s_cnt[D], s_run[D], s_tile[D], s_trun[D];
   __shared__ unsigned wrun[kBucketWaves][D];
@@ -449,22 +467,28 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(
     total += red[1][w];
   }
   const unsigned S = totals[b];
-  // A tile's slots: wave w owns the w-th contiguous eighth, walked in 64-slot
-  // rounds, so (wave, round, lane) is slot order.
+  // A tile's slots: each wave owns as many consecutive 64-slot rounds as
+  // spread the tile evenly, so (wave, round, lane) is slot order.  (With an
+  // eighth of the capacity each, a bucket of 4.3 K slots left half the waves idle
+  // and the others 16 rounds: 16.6 -> 14.3 us for 363 buckets.)
   unsigned key[kBucketItems], rank[kBucketItems];
   int val[kBucketItems];
   bool act[kBucketItems];
   unsigned *my = wrun[wave];
   // loads from clamped indices, all issued before any is used (see the
   // upsweep); an empty bucket loads nothing
+  unsigned rounds = 0;
   auto load_tile = [&](unsigned t0, bool vals) {
+    const unsigned n = S - t0 < (unsigned)TILE ? S - t0 : (unsigned)TILE;
+    rounds = (n + kBucketBlock - 1) / kBucketBlock;
 #pragma unroll
     for (int i = 0; i < kBucketItems; ++i) {
-      const unsigned e = t0 + (unsigned)(wave * PER_WAVE + i * kWave + lane);
-      act[i] = e < S;
+      const unsigned e = t0 + (wave * rounds + i) * kWave + lane;
+      act[i] = (unsigned)i < rounds && e < S;
+      if ((unsigned)i >= rounds) continue;  // uniform
       const unsigned ec = bs + (e < S ? e : S - 1);
-      key[i] = S > 0 ? kin[ec] : 0u;
-      if (vals) val[i] = S > 0 ? vin[ec] : 0;
+      key[i] = kin[ec];
+      if (vals) val[i] = vin[ec];
     }
   };
   // Stable ranks of the tile in registers among its equal low digits, per
@@ -472,6 +496,7 @@ __global__ __launch_bounds__(kBucketBlock) void bucket_sort_kernel(
   auto rank_tile = [&]() {
 #pragma unroll
     for (int i = 0; i < kBucketItems; ++i) {
+      if ((unsigned)i >= rounds) continue;  // uniform
       const unsigned d = key[i] & (D - 1);
       const uint64_t peers = match_digit<SB>(d, act[i]);
       if (act[i]) rank[i] = my[d] + (unsigned)popc_below(peers);
@@ -591,7 +616,7 @@ int run_high_pass(const SlotKey &sk, int64_t M, int shift, unsigned *kout, int *
 // Workspace: two key/position buffer pairs (ping-pong), the histograms and
 // the digit totals (the active-slot count is their sum).
 size_t slot_sort_workspace(int64_t M) {
-  const int64_t ntiles = ceil_div(std::max<int64_t>(M, 1), kSortTile);
+  const int64_t ntiles = max_sort_tiles(M);
   return 4 * align256((size_t)M * 4) + align256((size_t)(kMaxRadix * ntiles) * 4) + align256(kMaxRadix * 4);
 }
 
@@ -624,9 +649,8 @@ int slot_sort(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, i
   const size_t a = align256((size_t)M * 4);
   unsigned *kbuf[2] = {reinterpret_cast<unsigned *>(w), reinterpret_cast<unsigned *>(w + 2 * a)};
   int *vbuf[2] = {reinterpret_cast<int *>(w + a), reinterpret_cast<int *>(w + 3 * a)};
-  const int max_tiles = (int)ceil_div(std::max<int64_t>(M, 1), kSortTile);
-  const bool big = M > kBigSort;
-  const int ntiles = (int)ceil_div(std::max<int64_t>(M, 1), (int64_t)kBlock * (big ? kSortItemsBig : kSortItems));
+  const int64_t max_tiles = max_sort_tiles(M);
+  const int ntiles = sort_tiles(M);
   unsigned *hist = reinterpret_cast<unsigned *>(w + 4 * a);
   unsigned *totals = reinterpret_cast<unsigned *>(w + 4 * a + align256((size_t)(kMaxRadix * max_tiles) * 4));
   const unsigned nkeys = (unsigned)((int64_t)nchunks * N);
@@ -634,12 +658,12 @@ int slot_sort(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, i
   int rb, passes;
   sort_passes(nkeys, rb, passes);
   int rc;
-  if (big)
-    rc = rb == 9 ? run_passes<9, kSortItemsBig>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s)
-                 : run_passes<8, kSortItemsBig>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s);
+  if (sort_big(M))
+    rc = rb == 9 ? run_passes<9, kBigItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s)
+                 : run_passes<8, kBigItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s);
   else
-    rc = rb == 9 ? run_passes<9, kSortItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s)
-                 : run_passes<8, kSortItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s);
+    rc = rb == 9 ? run_passes<9, kSmallItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s)
+                 : run_passes<8, kSmallItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s);
   if (rc != SFT_OK) return rc;
   *keys_sorted = kbuf[(passes - 1) & 1];
   *pos_sorted = vbuf[(passes - 1) & 1];
@@ -676,19 +700,17 @@ struct BucketBufs {
   int *v1, *v2;
   unsigned *hist, *totals;
   int ntiles, sb, rb;
-  bool big;
 };
 static int bucket_bufs(void *ws, int64_t M, int64_t N, int nchunks, BucketBufs &bb) {
   char *w = static_cast<char *>(ws);
   const size_t a = align256((size_t)M * 4);
-  const int max_tiles = (int)ceil_div(std::max<int64_t>(M, 1), kSortTile);
+  const int64_t max_tiles = max_sort_tiles(M);
   bb.k1 = reinterpret_cast<unsigned *>(w);
   bb.v1 = reinterpret_cast<int *>(w + a);
   bb.v2 = reinterpret_cast<int *>(w + 3 * a);
   bb.hist = reinterpret_cast<unsigned *>(w + 4 * a);
   bb.totals = reinterpret_cast<unsigned *>(w + 4 * a + align256((size_t)(kMaxRadix * max_tiles) * 4));
-  bb.big = M > kBigSort;
-  bb.ntiles = (int)ceil_div(std::max<int64_t>(M, 1), (int64_t)kBlock * (bb.big ? kSortItemsBig : kSortItems));
+  bb.ntiles = sort_tiles(M);
   if (!bucket_plan((int64_t)nchunks * N, bb.sb, bb.rb)) return fail(SFT_EINVAL, "slot bucket sort: key space too large");
   return SFT_OK;
 }
@@ -705,10 +727,10 @@ int slot_sort_buckets_high(const int32_t *idx, int64_t M, int K, int64_t N, int 
   const SlotKey sk{idx, idx1 ? idx1 : idx, idx1 ? M / 2 : M, (unsigned)N, FastDiv((uint32_t)K),
                    FastDiv((uint32_t)chunk_rows), nkeys};
 #define SFT_HIGH_PASS(RB)                                                                                          \
-  rc = bb.big ? run_high_pass<RB, kSortItemsBig>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles, clear, \
-                                                 nclear, s)                                                        \
-              : run_high_pass<RB, kSortItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles, clear,    \
-                                              nclear, s)
+  rc = sort_big(M) ? run_high_pass<RB, kBigItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,      \
+                                                  clear, nclear, s)                                               \
+                   : run_high_pass<RB, kSmallItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,    \
+                                                    clear, nclear, s)
   if (bb.rb == 8) SFT_HIGH_PASS(8);
   else if (bb.rb == 9) SFT_HIGH_PASS(9);
   else SFT_HIGH_PASS(10);

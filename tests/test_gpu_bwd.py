@@ -112,6 +112,22 @@ def test_sorted_bwd_tile_groups(B, N, K, L, hot):
     assert rel_err(db, G.astype(np.float64).sum(0)) <= 1e-5
 
 
+@pytest.mark.parametrize("B,N,K", [
+    (1024, 129, 1), (205, 300, 5),      # one sort tile of 1024 slots, one slot more
+    (4096, 128, 2), (4097, 128, 2),     # one bucket of 8192 slots, one tile; two slots more
+    (16384, 700, 32), (16385, 700, 32),  # the last batch of 1024-slot tiles, the first of 4096-slot ones
+    (700, 300000, 33),                  # radix passes only (keys beyond the buckets)
+    (16400, 280000, 33),                # the same with the larger tiles
+])
+def test_sorted_bwd_sort_tile_edges(B, N, K):
+    announce(f"bwd sort tile edges B={B} N={N} K={K}")
+    g = np.random.default_rng(B + N)
+    idx = g.integers(0, N, (B, K)).astype(np.int32)  # every slot active
+    G = g.standard_normal((B, 8)).astype(np.float32)
+    dW, _ = run_bwd(idx, G, N, _native.SFT_BWD_OVERWRITE)
+    assert np.array_equal(dW, ft_oracle.bwd_f32(idx, G, N)[0])
+
+
 @pytest.mark.parametrize("N", [2500, 1500])
 def test_sorted_bwd_every_segment_long(N):
     """Every feature long (~450 and ~750 slots per position chunk): thousands
