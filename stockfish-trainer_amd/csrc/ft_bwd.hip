@@ -1191,6 +1191,13 @@ __device__ __forceinline__ f32x4 shfl_xor4(f32x4 v, int m) {
   return f32x4{__shfl_xor(v.x, m), __shfl_xor(v.y, m), __shfl_xor(v.z, m), __shfl_xor(v.w, m)};
 }
 
+// NT: non-temporal stores of the grad tiles, for batches whose tiles of both
+// perspectives outgrow the 256 MB MALL: storing them through it pushed out lines
+// that the gathers read.  The input stage of L1 = 1040, both ways, plain / NT:
+// 65 536 positions 1627 / 1608 us, 50 000 1339 / 1329, 40 000 1183 / 1171, 20 000
+// 727 / 728; L1 = 512, 50 000 704 / 702.
+constexpr int64_t kEpiNtBytes = 256ll << 20;
+template <bool NT>
 __global__ __launch_bounds__(kBlock) void bwd_epilogue_kernel(BwdEpilogue e, ColMap map, int64_t B, int ntiles) {
   __shared__ f32x4 red[kWavesPerBlock][kEpiIt][kWave];
   const int wave = uniform(threadIdx.x / kWave);
@@ -1252,7 +1259,7 @@ __global__ __launch_bounds__(kBlock) void bwd_epilogue_kernel(BwdEpilogue e, Col
               const int64_t kq = 4 * (int64_t)(colm[i] - 2 * map.half4);  // PSQT column of element 0
               if (k >= kq && k < kq + 4) d[(int)(k - kq)] = 0.0f + (p == 0 ? dp : -dp);
             }
-            gt[((int64_t)tile[i] * B + b) * kBwdTileCh + q] = d;
+            store_row<NT>(gt + ((int64_t)tile[i] * B + b) * kBwdTileCh + q, d);
           }
           bsum[i] += d;
         }
@@ -2163,8 +2170,9 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   if (!forked) side_join.release();
   {
     ProfScope prof(kProfBwdEpilogue, s);
-    hipLaunchKernelGGL(bwd_epilogue_kernel, dim3((unsigned)lay.nparts), dim3(kBlock), 0, s, e, map, B,
-                       map_tiles(map));
+    const bool nt_tiles = 2 * (int64_t)map_tiles(map) * B * 16 * kBwdTileCh > kEpiNtBytes;
+    hipLaunchKernelGGL(nt_tiles ? bwd_epilogue_kernel<true> : bwd_epilogue_kernel<false>, dim3((unsigned)lay.nparts),
+                       dim3(kBlock), 0, s, e, map, B, map_tiles(map));
     if ((rc = check_launch("epilogue backward")) != SFT_OK) return rc;
   }
   // the bias reduction rides in perspective 0's first gather launch
