@@ -29,15 +29,14 @@ namespace {
 // large one pays per tile, for its digit counts and the scans that walk them,
 // and shares the GPU: 2.1 M slots, both perspectives' steps with 4 / 8 / 16 per
 // thread, L = 136 387 / 369 / 366 us, L = 1048 1668 / 1645 / 1634 us.
+// (The count buffer has 2^10 counts per 2048 slots, which 1024-slot tiles fill
+// with 9-bit digits; 10-bit ones keep the large tiles.)
 constexpr int64_t kSmallSlots = 1 << 19;
 constexpr int kSmallItems = 4, kBigItems = 16;
-inline bool sort_big(int64_t M) { return M > kSmallSlots; }
-inline int sort_tiles(int64_t M) {
-  return (int)ceil_div(std::max<int64_t>(M, 1), (int64_t)kBlock * (sort_big(M) ? kBigItems : kSmallItems));
-}
-// The count buffer's tiles: at least sort_tiles(M), and growing with M.
-inline int64_t max_sort_tiles(int64_t M) {
-  return std::max<int64_t>(sort_tiles(M), sort_tiles(std::min(M, kSmallSlots)));
+constexpr int kSortTile = 2048;  // sizes the count buffer
+inline bool sort_big(int64_t M, int rb) { return M > kSmallSlots || rb > 9; }
+inline int sort_tiles(int64_t M, int rb) {
+  return (int)ceil_div(std::max<int64_t>(M, 1), (int64_t)kBlock * (sort_big(M, rb) ? kBigItems : kSmallItems));
 }
 constexpr int kMaxRadix = 1024;  // 10-bit digits (the bucket sort's first pass)
 #ifndef SFT_SORT_BUCKETS
@@ -616,7 +615,7 @@ int run_high_pass(const SlotKey &sk, int64_t M, int shift, unsigned *kout, int *
 // Workspace: two key/position buffer pairs (ping-pong), the histograms and
 // the digit totals (the active-slot count is their sum).
 size_t slot_sort_workspace(int64_t M) {
-  const int64_t ntiles = max_sort_tiles(M);
+  const int64_t ntiles = ceil_div(std::max<int64_t>(M, 1), kSortTile);
   return 4 * align256((size_t)M * 4) + align256((size_t)(kMaxRadix * ntiles) * 4) + align256(kMaxRadix * 4);
 }
 
@@ -649,16 +648,16 @@ int slot_sort(const int32_t *idx, int64_t M, int K, int64_t N, int chunk_rows, i
   const size_t a = align256((size_t)M * 4);
   unsigned *kbuf[2] = {reinterpret_cast<unsigned *>(w), reinterpret_cast<unsigned *>(w + 2 * a)};
   int *vbuf[2] = {reinterpret_cast<int *>(w + a), reinterpret_cast<int *>(w + 3 * a)};
-  const int64_t max_tiles = max_sort_tiles(M);
-  const int ntiles = sort_tiles(M);
+  const int64_t max_tiles = ceil_div(std::max<int64_t>(M, 1), kSortTile);
   unsigned *hist = reinterpret_cast<unsigned *>(w + 4 * a);
   unsigned *totals = reinterpret_cast<unsigned *>(w + 4 * a + align256((size_t)(kMaxRadix * max_tiles) * 4));
   const unsigned nkeys = (unsigned)((int64_t)nchunks * N);
   const SlotKey sk{idx, idx, M, (unsigned)N, FastDiv((uint32_t)K), FastDiv((uint32_t)chunk_rows), nkeys};
   int rb, passes;
   sort_passes(nkeys, rb, passes);
+  const int ntiles = sort_tiles(M, rb);
   int rc;
-  if (sort_big(M))
+  if (sort_big(M, rb))
     rc = rb == 9 ? run_passes<9, kBigItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s)
                  : run_passes<8, kBigItems>(sk, M, passes, kbuf, vbuf, hist, totals, ntiles, clear, nclear, s);
   else
@@ -704,14 +703,14 @@ struct BucketBufs {
 static int bucket_bufs(void *ws, int64_t M, int64_t N, int nchunks, BucketBufs &bb) {
   char *w = static_cast<char *>(ws);
   const size_t a = align256((size_t)M * 4);
-  const int64_t max_tiles = max_sort_tiles(M);
+  const int64_t max_tiles = ceil_div(std::max<int64_t>(M, 1), kSortTile);
   bb.k1 = reinterpret_cast<unsigned *>(w);
   bb.v1 = reinterpret_cast<int *>(w + a);
   bb.v2 = reinterpret_cast<int *>(w + 3 * a);
   bb.hist = reinterpret_cast<unsigned *>(w + 4 * a);
   bb.totals = reinterpret_cast<unsigned *>(w + 4 * a + align256((size_t)(kMaxRadix * max_tiles) * 4));
-  bb.ntiles = sort_tiles(M);
   if (!bucket_plan((int64_t)nchunks * N, bb.sb, bb.rb)) return fail(SFT_EINVAL, "slot bucket sort: key space too large");
+  bb.ntiles = sort_tiles(M, bb.rb);
   return SFT_OK;
 }
 
@@ -727,7 +726,7 @@ int slot_sort_buckets_high(const int32_t *idx, int64_t M, int K, int64_t N, int 
   const SlotKey sk{idx, idx1 ? idx1 : idx, idx1 ? M / 2 : M, (unsigned)N, FastDiv((uint32_t)K),
                    FastDiv((uint32_t)chunk_rows), nkeys};
 #define SFT_HIGH_PASS(RB)                                                                                          \
-  rc = sort_big(M) ? run_high_pass<RB, kBigItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,      \
+  rc = sort_big(M, RB) ? run_high_pass<RB, kBigItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,      \
                                                   clear, nclear, s)                                               \
                    : run_high_pass<RB, kSmallItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,    \
                                                     clear, nclear, s)
