@@ -1426,11 +1426,14 @@ int fwd_f32(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int
   // launch still has waves for every CU and each keeps 16 (8) rows in flight:
   // a position's rows are one chain of U-row steps, each a memory round trip
   // (L = 1048: B = 256, K = 32 12.4 -> 5.9 us; B = 64, K = 160 46 -> 14 us).
-  const int few = vec ? few_positions_cpl(B, cols) : 0;
+  // Their lists end on whole U-row steps; where that does not fit the LDS lists
+  // (K from 4081, of the 4092 that do) the general mapping stays.
+  const int kpad16 = (K + 15) / 16 * 16;
+  const int few = vec && index_lds_bytes(kWave, kpad16) <= kMaxIndexLds ? few_positions_cpl(B, cols) : 0;
   if (few > 0) m = Mapping{kWave, few, (int)ceil_div(cols, (int64_t)kWave * few)};
   const int ppb = kWavesPerBlock * (kWave / m.G);
   const dim3 grid((unsigned)ceil_div(B, ppb), (unsigned)m.slabs);
-  const int kpad = few > 0 ? (K + 15) / 16 * 16 : round_up4(K);  // whole U-row steps of a list
+  const int kpad = few > 0 ? kpad16 : round_up4(K);
   const size_t lds = index_lds_bytes(m.G, kpad);
   if (lds > kMaxIndexLds) return fail(SFT_EUNSUPPORTED, "sft_ft_fwd_f32: max_active too large for the LDS index lists");
   ProfScope prof(kProfFwdF32, s);

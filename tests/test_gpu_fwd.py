@@ -73,6 +73,21 @@ def test_fwd_rows_few_positions(B, N, K, L):
     assert np.array_equal(host(out), ft_oracle.fwd_f32(idx, W, b))
 
 
+# 64 KB of LDS lists hold 4092 slots a position, 4080 of them in whole 16-slot steps
+@pytest.mark.parametrize("K", [4080, 4081, 4092, 4093])
+def test_fwd_rows_longest_lists(K):
+    announce(f"fwd rows, longest lists K={K}")
+    B, N, L = 9, 4200, 256
+    idx, W, b, _ = case(K, B, N, K, L)
+    out = torch.empty(B, L, device=DEV)
+    if K == 4093:
+        with pytest.raises(RuntimeError, match="max_active too large"):
+            _native.ft_fwd_f32(dev(idx), dev(W), dev(b), out, rows=True)
+        return
+    _native.ft_fwd_f32(dev(idx), dev(W), dev(b), out, rows=True)
+    assert np.array_equal(host(out), ft_oracle.fwd_f32(idx, W, b))
+
+
 def test_fwd_repeated_feature_and_last_row():
     announce("fwd repeated features, index N-1")
     N, L = 40, 64
