@@ -1408,39 +1408,28 @@ size_t index_lds_bytes(int G, int K) {
   return (size_t)(kWavesPerBlock * ppw * round_up4(K) + kWavesPerBlock * ppw) * sizeof(int);
 }
 
-// Chunks per lane of the row gather's few-position mapping, 0 for the general one.
-constexpr int64_t kFewWaves = 8192;  // 8 per SIMD: as many as run at once
-static int few_positions_cpl(int64_t B, int64_t cols) {
-  if (B * ceil_div(cols, (int64_t)kWave) <= kFewWaves) return 1;
-  if (B * ceil_div(cols, (int64_t)2 * kWave) <= kFewWaves) return 2;
-  return 0;
-}
-
 int fwd_f32(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int L, const float *bias, float *out,
             hipStream_t s) {
   const bool vec = (L % 4 == 0) && ((uintptr_t)W % 16 == 0) && ((uintptr_t)bias % 16 == 0) &&
                    ((uintptr_t)out % 16 == 0);
   const int64_t cols = vec ? L / 4 : L;
   Mapping m = choose_mapping(cols);
-  // Few positions: a wave per position and 64 or 128 chunks of it, so that the
-  // launch still has waves for every CU and each keeps 16 (8) rows in flight:
-  // a position's rows are one chain of U-row steps, each a memory round trip
-  // (L = 1048: B = 256, K = 32 12.4 -> 5.9 us; B = 64, K = 160 46 -> 14 us).
-  // Their lists end on whole U-row steps; where that does not fit the LDS lists
-  // (K from 4081, of the 4092 that do) the general mapping stays.
+  // Few positions (few_positions): a wave per position and 64 chunks, 16 rows in
+  // flight.  Their lists end on whole 16-row steps; where that does not fit the
+  // LDS lists (K from 4081, of the 4092 that do) the general mapping stays.
   const int kpad16 = (K + 15) / 16 * 16;
-  const int few = vec && index_lds_bytes(kWave, kpad16) <= kMaxIndexLds ? few_positions_cpl(B, cols) : 0;
-  if (few > 0) m = Mapping{kWave, few, (int)ceil_div(cols, (int64_t)kWave * few)};
+  const bool few = vec && few_positions(B, K, cols) && index_lds_bytes(kWave, kpad16) <= kMaxIndexLds;
+  if (few) m = Mapping{kWave, 1, (int)ceil_div(cols, (int64_t)kWave)};
   const int ppb = kWavesPerBlock * (kWave / m.G);
   const dim3 grid((unsigned)ceil_div(B, ppb), (unsigned)m.slabs);
-  const int kpad = few > 0 ? kpad16 : round_up4(K);
+  const int kpad = few ? kpad16 : round_up4(K);
   const size_t lds = index_lds_bytes(m.G, kpad);
   if (lds > kMaxIndexLds) return fail(SFT_EUNSUPPORTED, "sft_ft_fwd_f32: max_active too large for the LDS index lists");
   ProfScope prof(kProfFwdF32, s);
-  if (few > 0) {
-    hipLaunchKernelGGL((few == 1 ? fwd_f32_kernel<f32x4, 64, 1, 16> : fwd_f32_kernel<f32x4, 64, 2, 8>), grid,
-                       dim3(kBlock), lds, s, idx, B, K, (int)N, reinterpret_cast<const f32x4 *>(W), cols,
-                       reinterpret_cast<const f32x4 *>(bias), reinterpret_cast<f32x4 *>(out), kpad);
+  if (few) {
+    hipLaunchKernelGGL((fwd_f32_kernel<f32x4, 64, 1, 16>), grid, dim3(kBlock), lds, s, idx, B, K, (int)N,
+                       reinterpret_cast<const f32x4 *>(W), cols, reinterpret_cast<const f32x4 *>(bias),
+                       reinterpret_cast<f32x4 *>(out), kpad);
   } else if (vec) {
     SFT_G_CASES(launch_fwd_f32, f32x4, grid, lds, s, idx, B, K, (int)N, W, cols, bias, out, kpad)
   } else {

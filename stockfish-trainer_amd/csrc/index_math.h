@@ -52,6 +52,27 @@ struct FastDiv {
   }
 };
 
+// ---- the row gather's mapping of few positions ----
+// Whether B positions of `cols` 16-byte row chunks and K slots are gathered by a
+// wave per position and 64 chunks, 16 rows in flight, instead of the general
+// mapping (as many positions per wave as its rows are narrow, 4 rows in flight).
+// A position's rows are one chain of memory round trips, so the few-position
+// mapping wins while the launch is latency and loses once the rows' bytes, or
+// for narrow rows the waves themselves, are what takes the time.  General /
+// few-position, us (N = 23 232, K = 32; N = 85 296, K = 160 likewise by L, B):
+//   K = 32:  L = 32: 1024 6.4 / 4.8, 2048 6.2 / 5.5, 2560 6.2 / 6.5, 8192 6.2 / 11.6
+//            L = 256: 1024 7.7 / 6.3, 2048 9.7 / 9.2, 4096 14.4 / 15.2
+//            L = 520: 1024 15.0 / 11.3, 2048 19.3 / 19.5, 3072 25.4 / 27.2
+//            L = 1048: 256 13.7 / 7.6, 1024 19.8 / 18.7, 2048 32.9 / 33.6
+//   K = 160: L = 64: 3072 28.9 / 20.3, 8192 33.6 / 43.5;  L = 256: 1536 31.0 / 29.3, 2560 43.6 / 45.4
+//            L = 520: 1024 56 / 44, 1536 63 / 67;  L = 1048: 512 64 / 46, 1024 82 / 86
+SFT_HD inline bool few_positions(int64_t B, int K, int64_t cols) {
+  if (cols > 1 << 21) return false;  // a launch's column slabs stay below 2^16
+  if (K <= 32) return B <= 2048;
+  const int64_t most = (1 << 17) / cols;
+  return B <= (most < 768 ? 768 : most > 3072 ? 3072 : most);
+}
+
 // ---- XCD-aware tile schedule ----
 // MI355X runs a dispatch's workgroups round-robin over its 8 XCDs (workgroup i
 // on XCD i % 8), and each XCD has its own 4 MB L2.  Tiled kernels give every

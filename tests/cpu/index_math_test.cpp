@@ -195,7 +195,27 @@ static void check_chunk0_buckets(int64_t N, int nchunks, int sb) {
         (long long)(N >> sb));
 }
 
+// The row gather's few-position mapping, on both sides of its line: rows of one
+// 64-lane slab and of several, K up to 32 and above (16-byte chunks per row).
+static void check_few_positions() {
+  struct Case {
+    int64_t B;
+    int K;
+    int64_t cols;
+    bool few;
+  };
+  for (const Case &c : {Case{1, 32, 8, true}, Case{2048, 32, 8, true}, Case{2049, 32, 8, false},
+                        Case{8192, 32, 8, false}, Case{8192, 32, 32, false}, Case{4096, 32, 130, false},
+                        Case{256, 32, 262, true}, Case{2048, 32, 512, true}, Case{3072, 160, 16, true},
+                        Case{4097, 160, 16, false}, Case{8192, 160, 32, false}, Case{2048, 160, 64, true},
+                        Case{2560, 160, 64, false}, Case{1008, 160, 130, true}, Case{1536, 160, 130, false},
+                        Case{768, 160, 262, true}, Case{1024, 160, 262, false}, Case{512, 160, 512, true},
+                        Case{256, 4080, 1 << 20, true}, Case{1, 8, (1 << 21) + 1, false}})
+    CHECK(few_positions(c.B, c.K, c.cols) == c.few, "B=%lld K=%d cols=%lld", (long long)c.B, c.K, (long long)c.cols);
+}
+
 int main() {
+  check_few_positions();
   // the sort divides slot numbers by max_active (K) and positions by the
   // position-chunk rows (ceil(B / 2) or B); cover every K the ABI allows up to
   // 4096, the workloads' batches and chunk sizes, and powers of two
