@@ -1033,8 +1033,13 @@ __global__ __launch_bounds__(kBlock) void bwd_pair_gather_kernel(TiledArgs a) {
 // 23 232, 32, 1048: 256 84 / 56, 2904 92 / 86, 4356 97 / 105;  520: 2904 72 / 63,
 // 5808 78 / 81;  85 296, 160, 1048: 2132 204 / 173, 3198 224 / 226;  4096, 32,
 // 1048: 512 55 / 47, 1536 59 / 58;  517: even.
-bool few_slots(int64_t B, int K, int64_t N) {
-  return B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) && B * (int64_t)K <= 4 * N;
+// A grad that is not 16-byte aligned keeps the tiles: its row gather reads floats
+// and leaves each long segment to one lane group (2904 positions of Zipf(1.1)
+// rows, N = 23 232: L = 1048 tiled 120, rows 272 us, L = 520 88 / 231; uniform rows
+// 93 / 78).
+bool few_slots(int64_t B, int K, int64_t N, const float *grad) {
+  return B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) && B * (int64_t)K <= 4 * N &&
+         (uintptr_t)grad % 16 == 0;
 }
 
 // Long-segment slots per tile of a gather over so many slots: at most
@@ -1699,7 +1704,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
   // The tiled weight-grad gather reads the grad in column tiles; the bias pass
   // writes that layout while it streams the grad (16-byte loads when the grad
   // allows them, 4-byte loads otherwise), and stores 16-byte weight-grad chunks.
-  const bool tiled = !(flags & SFT_BWD_ATOMIC) && M > 0 && tiled_shape(B, L, flags) && !few_slots(B, K, N) &&
+  const bool tiled = !(flags & SFT_BWD_ATOMIC) && M > 0 && tiled_shape(B, L, flags) && !few_slots(B, K, N, grad) &&
                      (uintptr_t)dW % 16 == 0;
   f32x4 *gt = tiled ? reinterpret_cast<f32x4 *>(w + lay.gt) : nullptr;
 

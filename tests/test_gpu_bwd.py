@@ -363,6 +363,30 @@ def test_bwd_unaligned_grad_keeps_the_tiled_gather(offset):
     assert rel_err(host(db), G.astype(np.float64).sum(0)) <= 1e-5
 
 
+@pytest.mark.parametrize("offset,tiled", [(0, False), (1, True), (4, False)])
+def test_bwd_few_slots_unaligned_grad_keeps_the_tiled_gather(offset, tiled):
+    """Up to four slots a feature the row gather runs, unless the grad is not
+    16-byte aligned: its rows would be summed a float at a time, hot features'
+    in one lane group (here feature 3, in every position)."""
+    announce(f"bwd few slots, unaligned grad offset={offset}")
+    B, N, K, L = 700, 800, 4, 136
+    idx, _, _, G = case(34, B, N, K, L)
+    idx[:, 1] = 3
+    dW = torch.full((N, L), float("nan"), device=DEV)
+    db = torch.full((L,), float("nan"), device=DEV)
+    g, i = _unaligned(dev(G), offset), dev(idx)
+    _native.prof_enable(True)
+    try:
+        _native.prof_collect()
+        _native.ft_bwd_f32(i, dW, db, g, _native.SFT_BWD_OVERWRITE)
+        ran = {k: n for k, (_, n) in _native.prof_collect().items()}
+    finally:
+        _native.prof_enable(False)
+    assert (ran.get("bwd_tiled_gather", 0) > 0, ran.get("bwd_feature_gather", 0) > 0) == (tiled, not tiled)
+    assert np.array_equal(host(dW), ft_oracle.bwd_f32(idx, G, N)[0])
+    assert rel_err(host(db), G.astype(np.float64).sum(0)) <= 1e-5
+
+
 def test_prepared_bwd_no_active_slots():
     announce("prepared bwd, every slot inactive")
     idx = np.full((50, 8), -1, np.int32)
