@@ -1890,9 +1890,8 @@ struct PairLayout {
 };
 
 // Batches whose two grad tiles fit an XCD's L2 together (B <= 16 384).
-bool pair_one_launch(int64_t B, int64_t N) {
-  return 2 * B * 16 * kBwdTileCh <= (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) && slot_sort_buckets_supported(N, 2);
-}
+constexpr int64_t kPairOneLaunchBatch = (int64_t)(SFT_BWD_ONE_CHUNK_BYTES) / (2 * 16 * kBwdTileCh);
+bool pair_one_launch(int64_t B, int64_t N) { return B <= kPairOneLaunchBatch && slot_sort_buckets_supported(N, 2); }
 
 void make_pair_layout(int64_t B, int K, int64_t N, int L, PairLayout &lay) {
   const int64_t M = B * K;
@@ -1929,10 +1928,14 @@ void make_pair_layout(int64_t B, int K, int64_t N, int L, PairLayout &lay) {
   lay.total = off;
 }
 
+// At least what every smaller batch needs: callers size one workspace for their
+// largest batch.  (The one-launch layout holds both perspectives' grad tiles, the
+// layout above it one and the carried sums of N rows, which for few rows is less.)
 size_t bwd_pair_workspace(int64_t B, int K, int64_t N, int L) {
-  PairLayout lay;
+  PairLayout lay, most;
   make_pair_layout(B, K, N, L, lay);
-  return lay.total;
+  make_pair_layout(std::min<int64_t>(B, kPairOneLaunchBatch), K, N, L, most);
+  return std::max(lay.total, most.total);
 }
 
 // One perspective's slots sorted, with their segments (on the side stream).

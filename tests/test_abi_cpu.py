@@ -254,6 +254,28 @@ def rank_lists_bytes(B, K):
     return _a256(bp * kpad * 4) + 2 * _a256(bp * 4) + 2 * _a256(bp * 16)
 
 
+@pytest.mark.parametrize("N", [500, 3000, 24576, 140000])
+@pytest.mark.parametrize("K", [4, 32, 160])
+@pytest.mark.parametrize("L", [264, 1048])
+def test_backward_workspaces_hold_smaller_batches(N, K, L):
+    """A workspace sized for a program's largest batch serves its smaller ones."""
+    lib = _native.lib()
+    most = None
+    for B in (1, 256, 2048, 4096, 8192, 16384, 16385, 20000, 32768, 32769, 40000, 65536):
+        need = []
+        f, b, s = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
+        assert lib.sft_ft_pair_workspace_size(B, K, 1, _i64s(N), _i64s(0), L, ctypes.byref(f), ctypes.byref(b)) == 0
+        need += [f.value, b.value]
+        assert lib.sft_ft_transform_workspace_size(B, K, 1, _i64s(N), _i64s(0), L, L - 8, ctypes.byref(f),
+                                                   ctypes.byref(b), ctypes.byref(s)) == 0
+        need += [f.value, b.value, s.value]
+        for flags in (_native.SFT_BWD_OVERWRITE, _native.SFT_BWD_OVERWRITE | _native.SFT_BWD_PREPARED):
+            assert lib.sft_ft_bwd_f32_workspace_size(B, K, N, L, flags, ctypes.byref(b)) == 0
+            need.append(b.value)
+        assert most is None or all(n >= m for n, m in zip(need, most)), (B, need, most)
+        most = need
+
+
 def test_pair_workspace_size_and_shape_checks():
     lib = _native.lib()
     fb, bb = ctypes.c_size_t(0), ctypes.c_size_t(0)
