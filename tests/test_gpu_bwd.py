@@ -115,6 +115,7 @@ def test_sorted_bwd_tile_groups(B, N, K, L, hot):
 @pytest.mark.parametrize("B,N,K", [
     (1024, 129, 1), (205, 300, 5),      # one sort tile of 1024 slots, one slot more
     (4096, 128, 2), (4097, 128, 2),     # one bucket of 8192 slots, one tile; two slots more
+    (2048, 128, 2), (2049, 128, 2),     # one bucket tile's first half (8 rounds of 512 slots), and into the second
     (16384, 700, 32), (16385, 700, 32),  # the last batch of 1024-slot tiles, the first of 4096-slot ones
     (700, 300000, 33),                  # radix passes only (keys beyond the buckets)
     (16400, 280000, 33),                # the same with the larger tiles
