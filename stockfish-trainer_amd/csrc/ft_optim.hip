@@ -76,11 +76,7 @@ constexpr int kOptRowChunks = 8;  // 16-byte chunks per lane kept in registers (
 
 // 2-D tables, cols % 4 == 0 and cols <= 4 * 64 * kOptRowChunks: one wave per row,
 // the whole row of all five tensors loaded into registers before the norm's
-// reduction, so the loads of a row are all in flight together.  Bound by HBM
-// (20 bytes read, 12 written per element); the five tensors outgrow every cache
-// at the tables' sizes, so loads and stores are non-temporal: 25 344 rows of
-// 1048 and the bias, tensors in turn from three sets, 173.5 -> 167.4 us
-// (4.9 -> 5.1 TB/s; the loads alone non-temporal 178.5 us, the stores alone 183).
+// reduction, so the loads of a row are all in flight together.
 template <int NCH>
 __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restrict__ p, const f32x4 *__restrict__ g,
                                                                  f32x4 *__restrict__ v, f32x4 *__restrict__ m,
@@ -97,11 +93,11 @@ __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restri
   for (int j = 0; j < NCH; ++j) {
     const int c = lane + kWave * j;
     const bool ok = c < cols4;
-    pr[j] = ok ? __builtin_nontemporal_load(p + base + c) : z;
-    gr[j] = ok ? __builtin_nontemporal_load(g + base + c) : z;
-    vr[j] = ok ? __builtin_nontemporal_load(v + base + c) : z;
-    mr[j] = ok ? __builtin_nontemporal_load(m + base + c) : z;
-    mpr[j] = ok ? __builtin_nontemporal_load(mp + base + c) : z;
+    pr[j] = ok ? p[base + c] : z;
+    gr[j] = ok ? g[base + c] : z;
+    vr[j] = ok ? v[base + c] : z;
+    mr[j] = ok ? m[base + c] : z;
+    mpr[j] = ok ? mp[base + c] : z;
   }
   float sq = 0.f;
 #pragma unroll
@@ -121,9 +117,9 @@ __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restri
       vv[e] = ve;
       mv[e] = me;
     }
-    __builtin_nontemporal_store(pv, p + base + c);
-    __builtin_nontemporal_store(vv, v + base + c);
-    __builtin_nontemporal_store(mv, m + base + c);
+    p[base + c] = pv;
+    v[base + c] = vv;
+    m[base + c] = mv;
   }
 }
 
