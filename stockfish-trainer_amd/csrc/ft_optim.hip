@@ -76,7 +76,13 @@ constexpr int kOptRowChunks = 8;  // 16-byte chunks per lane kept in registers (
 
 // 2-D tables, cols % 4 == 0 and cols <= 4 * 64 * kOptRowChunks: one wave per row,
 // the whole row of all five tensors loaded into registers before the norm's
-// reduction, so the loads of a row are all in flight together.
+// reduction, so the loads of a row are all in flight together.  Bound by HBM
+// (20 bytes read, 12 written per element).  Plain loads and stores: non-temporal
+// ones are faster only where such updates follow each other (25 344 rows of 1048,
+// three sets of tensors in turn 173 -> 168 us) and slower with a step's other
+// traffic between them, as in training (a 1 GB copy between updates: 24 576 x 1048
+// 152 -> 159 us, 60 720 x 1048 391 -> 411), and for smaller tables even in turn
+// (24 576 x 264 42 -> 48).
 template <int NCH>
 __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restrict__ p, const f32x4 *__restrict__ g,
                                                                  f32x4 *__restrict__ v, f32x4 *__restrict__ m,
