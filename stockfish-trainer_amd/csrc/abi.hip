@@ -42,7 +42,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
 int bwd_prep_bytes(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *bytes);
 int bwd_prepare(const int32_t *idx, int64_t B, int K, int64_t N, int L, uint32_t flags, void *prep,
                 size_t prep_bytes, hipStream_t s);
-bool sort_small(int64_t B, int K, int L);
+bool fwd_sort_in_line(int64_t B, int K, int64_t N, int L);
 size_t index_lds_bytes(int G, int K);
 int fwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, const FoldSrc &src, int64_t N, int L,
                  const float *bias, float *out0, float *out1, void *ws, size_t ws_bytes, hipStream_t s);
@@ -143,9 +143,9 @@ int fork_side(hipStream_t s, hipStream_t *side) {
   return SFT_OK;
 }
 
-int fork_sort(hipStream_t s, bool small, hipStream_t *side, bool *forked) {
-  *forked = !small;
-  if (small) {  // a captured fork costs the host nothing when it is replayed
+int fork_sort(hipStream_t s, bool in_line, hipStream_t *side, bool *forked) {
+  *forked = !in_line;
+  if (in_line) {  // a captured fork costs the host nothing when it is replayed
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     *forked = hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
   }
@@ -415,7 +415,7 @@ int sft_ft_fwd_f32_prep(const int32_t *idx, int64_t batch, int32_t max_active, c
                              workspace_bytes, flags, stream);
   hipStream_t side;
   bool forked;
-  int rc = fork_sort(s, sort_small(batch, max_active, output_size), &side, &forked);
+  int rc = fork_sort(s, fwd_sort_in_line(batch, max_active, num_inputs, output_size), &side, &forked);
   if (rc != SFT_OK) return rc;
   SideJoinGuard side_join(s);
   if (!forked) side_join.release();

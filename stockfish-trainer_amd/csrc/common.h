@@ -37,9 +37,9 @@ int check_launch(const char *what);
 // operations (event record / wait), so they capture into a graph like kernels.
 constexpr int kSideMarks = 2;
 int fork_side(hipStream_t s, hipStream_t *side);
-// fork_sort: fork_side, or for a sort too small for that to pay *side = s and
-// not *forked (nothing to join); under capture always a fork.
-int fork_sort(hipStream_t s, bool small, hipStream_t *side, bool *forked);
+// fork_sort: fork_side, or for a sort that goes in line (sort_in_line_fwd and its
+// neighbours) *side = s and not *forked (nothing to join); under capture always a fork.
+int fork_sort(hipStream_t s, bool in_line, hipStream_t *side, bool *forked);
 int mark_side(int slot);
 int wait_side(hipStream_t s, int slot);
 int join_side(hipStream_t s);

@@ -28,8 +28,8 @@
 
 namespace sft {
 
-bool sort_small(int64_t B, int K, int L);
 size_t index_lds_bytes(int G, int K);
+int table_parts(int64_t N);
 size_t slot_sort_workspace(int64_t M);
 // Stable sort of the active slots by (position chunk, feature); also zeroes
 // clear[0 .. nclear) before it returns (stream-ordered).
@@ -1602,7 +1602,6 @@ bool prep_pays(int64_t B, int K, int L, uint32_t flags) {
 #ifndef SFT_BWD_SPLIT_BUCKETS
 #define SFT_BWD_SPLIT_BUCKETS 1
 #endif
-constexpr int64_t kSmallSort = 1 << 16, kSmallSortNarrow = 1 << 21;  // slots (sort_small)
 constexpr int kChunk0Mark = 1;  // side-stream mark after chunk 0's buckets
 bool prep_split(int64_t B, int K, int64_t N, int L, uint32_t flags) {
   return prep_pays(B, K, L, flags) && (int64_t)K * SFT_BWD_SPLIT_K_PER_L >= L &&
@@ -1644,14 +1643,13 @@ int sort_and_segments(const int32_t *idx, int64_t B, int K, int64_t N, int nc, v
 
 }  // namespace
 
-// Whether a perspective's sort runs on the caller's stream: a fork and join
-// take about 27 us on the host, and a step whose launches take the host longer
-// than the GPU gains more from saving them than from the overlap.  Steps of both
-// perspectives launched eagerly, forked / in line, us: L = 1048 (N = 23 232), B = 300
-// 358 / 184, B = 2048 351 / 280, B = 4096 397 / 408; narrow rows (the split
-// prepared sort's), L = 136, B = 8192 417 / 271, B = 65 536 471 / 385.
-bool sort_small(int64_t B, int K, int L) {
-  return B * K <= ((int64_t)K * SFT_BWD_SPLIT_K_PER_L >= L ? kSmallSortNarrow : kSmallSort);
+// Rows narrow for their slot count (the split prepared sort's).
+static bool narrow_rows(int K, int L) { return (int64_t)K * SFT_BWD_SPLIT_K_PER_L >= L; }
+bool fwd_sort_in_line(int64_t B, int K, int64_t N, int L) {
+  return sort_in_line_fwd(B * K, K, L, narrow_rows(K, L), table_parts(N) == 1);
+}
+static bool bwd_sort_in_line(int64_t B, int K, int64_t N, int L, bool prepared) {
+  return sort_in_line_bwd(B * K, K, narrow_rows(K, L), prepared, table_parts(N) == 1);
 }
 
 int bwd_prep_bytes(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *bytes) {
@@ -1738,7 +1736,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
       // pass the forward left in the prepared buffer, into the workspace
       hipStream_t side;
       bool forked;
-      if ((rc = fork_sort(s, sort_small(B, K, L), &side, &forked)) != SFT_OK) return rc;
+      if ((rc = fork_sort(s, bwd_sort_in_line(B, K, N, L, true), &side, &forked)) != SFT_OK) return rc;
       if (forked) side_join.emplace(s);
       const SegBufs sbs = seg_bufs(seg, nc, N);
       const int64_t crow = nc > 1 ? half_rows(B) : B;
@@ -1766,7 +1764,7 @@ int bwd_f32(const int32_t *idx, int64_t B, int K, const float *grad, int64_t N, 
   } else if (sorted) {
     hipStream_t side;
     bool forked;
-    if ((rc = fork_sort(s, sort_small(B, K, L), &side, &forked)) != SFT_OK) return rc;
+    if ((rc = fork_sort(s, bwd_sort_in_line(B, K, N, L, false), &side, &forked)) != SFT_OK) return rc;
     if (forked) side_join.emplace(s);
     if ((rc = sort_and_segments(idx, B, K, N, nc, w + lay.sort, seg, &pos, side)) != SFT_OK) return rc;
   }
@@ -2012,10 +2010,10 @@ static int pair_sort_both(const int32_t *idx0, const int32_t *idx1, int64_t B, i
 // Both perspectives' slots in one sort on the side stream (key = perspective N +
 // feature, positions of perspective 1 from B on); joined by the caller when
 // *forked.
-static int pair_sort_once(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, int64_t N, char *sort_ws,
-                          int32_t *seg, SortedSlots &out, bool *forked, hipStream_t s) {
+static int pair_sort_once(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, int64_t N, int L, bool epilogue,
+                          char *sort_ws, int32_t *seg, SortedSlots &out, bool *forked, hipStream_t s) {
   hipStream_t side;
-  int rc = fork_sort(s, 2 * B * K <= 2 * kSmallSort, &side, forked);
+  int rc = fork_sort(s, sort_in_line_pair(B * K, N * L, epilogue), &side, forked);
   if (rc != SFT_OK) return rc;
   SideJoinGuard side_join(s);
   if (!*forked) side_join.release();
@@ -2064,8 +2062,8 @@ int bwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, con
   if (lay.one_launch) {
     f32x4 *gt1 = reinterpret_cast<f32x4 *>(w + lay.gt1);
     bool forked;
-    if ((rc = pair_sort_once(idx0, idx1, B, K, N, w + lay.sort[0], reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0],
-                             &forked, s)) != SFT_OK)
+    if ((rc = pair_sort_once(idx0, idx1, B, K, N, L, false, w + lay.sort[0],
+                             reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], &forked, s)) != SFT_OK)
       return rc;
     SideJoinGuard side_join(s);
     if (!forked) side_join.release();
@@ -2170,7 +2168,7 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   e.P = L - L1;
   SortedSlots ss[2];  // sorted on the side stream while the epilogue runs
   bool forked = true;
-  int rc = lay.one_launch ? pair_sort_once(idx0, idx1, B, K, N, w + lay.sort[0],
+  int rc = lay.one_launch ? pair_sort_once(idx0, idx1, B, K, N, L, true, w + lay.sort[0],
                                            reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], &forked, s)
                           : pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s);
   if (rc != SFT_OK) return rc;

@@ -1472,7 +1472,7 @@ static RankLists rank_lists_at(char *p, int64_t B, int K, int narrow) {
 #ifndef SFT_FWD_PART_BYTES
 #define SFT_FWD_PART_BYTES (7 << 19)
 #endif
-static int table_parts(int64_t N) {
+int table_parts(int64_t N) {
   const int64_t p = ceil_div(tile_rows(N) * (int64_t)kTileRowBytes, (int64_t)(SFT_FWD_PART_BYTES));
   return (int)std::min<int64_t>(std::max<int64_t>(p, 1), kMaxParts);
 }

@@ -73,6 +73,52 @@ SFT_HD inline bool few_positions(int64_t B, int K, int64_t cols) {
   return B <= (most < 768 ? 768 : most > 3072 ? 3072 : most);
 }
 
+// ---- which sorts run on the caller's stream ----
+// A sort of M = B K slots runs beside the kernels that do not need it, on a side
+// stream, or in line before them.  A fork and join cost the host about 27 us and
+// the GPU about 10 us; in line, nothing hides the sort's launches, most of which
+// fill few CUs.  So small sorts go in line, and the lines are where a step of
+// both perspectives takes as long either way (narrow: K >= L / 5, whose forward
+// runs the radix pass and whose backward the buckets; one_part: the table fits
+// one gather pass).  GPU time forked / in line with the host ahead, us; with the
+// host the slower one, short steps gain 50-100 us more by the sort in line.
+//
+// The prepared sort's part in the forward.  The more the gather moves, the more
+// it hides: for lists of more than 32 slots the line is on M L.
+//   K = 32, N = 23 232, L = 136: B = 16 384 173 / 159, 65 536 385 / 376, 100 000 548 / 537, 131 072
+//   741 / 725;  N = 85 296: 65 536 696 / 691, 131 072 1159 / 1169
+//   K = 64, N = 23 232, L = 264: 8192 235 / 238, 32 768 492 / 505, 65 536 898 / 921 (host-bound below
+//   24 000: 16 384 402 / 313);  K = 128, L = 520: 5000 378 / 394 (host-bound 408 / 386), 8000 468 / 484
+//   K = 160, N = 85 296, L = 136: 8192 391 / 384, 10 000 444 / 453;  L = 520: 1000 348 / 343, 3000 601 / 617;
+//   L = 800: 1000 469 / 462, 3000 811 / 828
+// Wide rows (the whole sort in the forward): K = 64, N = 23 232, L = 1048: 1000 238 / 227, 2048 347 / 348;
+// K = 32, L = 264: 6000 170 / 164, 12 000 192 / 194;  K = 160, N = 85 296, L = 1048: 64 442 / 443, 409 502 / 514.
+SFT_HD inline bool sort_in_line_fwd(int64_t M, int K, int L, bool narrow, bool one_part) {
+  if (!narrow) return M <= (one_part ? 1 << 16 : 1 << 14);
+  if (K > 32 && M * L > (one_part ? (int64_t)3 << 27 : (int64_t)3 << 26)) return false;
+  return M <= (one_part ? 3 << 20 : 1 << 21);
+}
+// The backward's: the buckets of a prepared sort, or (not prepared) the whole sort.
+// Buckets (the forward's part as above): K = 32, N = 23 232, L = 136: 65 536 387 / 376, 100 000 543 / 537,
+// 160 000 893 / 902;  N = 85 296: 65 536 705 / 691, 131 072 1161 / 1169;  K = 8, N = 4000, L = 32: 262 144
+// 439 / 438, 500 000 659 / 714;  K = 160, N = 85 296, L = 136: 8192 413 / 391, 16 384 576 / 555;
+// L = 264: 20 000 944 / 930.
+// Whole sort, one backward: L = 136, K = 32: 8192 57 / 47, 65 536 136 / 133, 131 072 260 / 265;
+// a step, L = 1048: 2048 258 / 251, 3000 310 / 316 (host-bound 358 / 316), 8192 407 / 414.
+SFT_HD inline bool sort_in_line_bwd(int64_t M, int K, bool narrow, bool prepared, bool one_part) {
+  if (!narrow) return M <= 1 << 16;
+  return M <= (!prepared || (K <= 32 && !one_part) ? 1 << 21 : 3 << 20);
+}
+// Both perspectives' sort of a composed backward over a table of so many values,
+// M slots each; epilogue: beside the post-FT epilogue's backward, which hides
+// more of it.  Host-bound steps (small tables) gain 40 us in line, the others
+// lose:  composed, N = 24 576, L = 1048, B = 2048 213 / 214 (host-bound 297 / 252);  N = 85 296: 545 / 550;
+// epilogue, N = 24 576: L = 264 141 / 148 (host-bound 324 / 290), L = 1048 375 / 384 (host-bound 379 / 389);
+// N = 85 296: L = 264 247 / 262 (host-bound 348 / 303), L = 1048 703 / 719.
+SFT_HD inline bool sort_in_line_pair(int64_t M, int64_t table, bool epilogue) {
+  return M <= 1 << 16 && table <= (epilogue ? 24 : 48) * (int64_t)1000000;
+}
+
 // ---- XCD-aware tile schedule ----
 // MI355X runs a dispatch's workgroups round-robin over its 8 XCDs (workgroup i
 // on XCD i % 8), and each XCD has its own 4 MB L2.  Tiled kernels give every

@@ -214,8 +214,46 @@ static void check_few_positions() {
     CHECK(few_positions(c.B, c.K, c.cols) == c.few, "B=%lld K=%d cols=%lld", (long long)c.B, c.K, (long long)c.cols);
 }
 
+// Which sorts run in line, on both sides of each line: positions, slots per
+// position, columns, narrow (K >= L / 5), the table in one part or several.
+static void check_sorts_in_line() {
+  struct Case {
+    int64_t B;
+    int K, L;
+    bool one_part, fwd, buckets, whole;
+  };
+  for (const Case &c : {
+           Case{300, 32, 136, true, true, true, true}, Case{65536, 32, 136, true, true, true, true},
+           Case{65537, 32, 136, true, true, true, false}, Case{98304, 32, 136, true, true, true, false},
+           Case{98305, 32, 136, true, false, false, false}, Case{65536, 32, 136, false, true, true, true},
+           Case{65537, 32, 136, false, false, false, false}, Case{393217, 8, 32, true, false, false, false},
+           Case{16384, 64, 264, true, true, true, true}, Case{32768, 64, 264, true, false, true, true},
+           Case{5000, 128, 520, true, true, true, true}, Case{8000, 128, 520, true, false, true, true},
+           Case{8192, 160, 136, false, true, true, true}, Case{10000, 160, 136, false, false, true, true},
+           Case{1000, 160, 520, false, true, true, true}, Case{3000, 160, 520, false, false, true, true},
+           Case{20000, 160, 264, false, false, false, false}, Case{19660, 160, 264, false, false, true, false},
+           // wide rows
+           Case{2048, 32, 1048, true, true, true, true}, Case{2049, 32, 1048, true, false, false, false},
+           Case{102, 160, 1048, false, true, true, true}, Case{103, 160, 1048, false, false, true, true}}) {
+    const bool narrow = 5 * c.K >= c.L;
+    const int64_t M = c.B * c.K;
+    CHECK(sort_in_line_fwd(M, c.K, c.L, narrow, c.one_part) == c.fwd, "fwd B=%lld K=%d L=%d", (long long)c.B, c.K, c.L);
+    CHECK(sort_in_line_bwd(M, c.K, narrow, true, c.one_part) == c.buckets, "buckets B=%lld K=%d L=%d", (long long)c.B,
+          c.K, c.L);
+    CHECK(sort_in_line_bwd(M, c.K, narrow, false, c.one_part) == c.whole, "whole B=%lld K=%d L=%d", (long long)c.B, c.K,
+          c.L);
+  }
+  for (bool epilogue : {false, true}) {  // N = 24 576 and 85 296 rows
+    CHECK(sort_in_line_pair(2048 * 32, 24576 * 264, epilogue) && !sort_in_line_pair(2049 * 32, 24576 * 264, epilogue),
+          "pair slots");
+    CHECK(sort_in_line_pair(65536, (int64_t)24576 * 1048, epilogue) == !epilogue, "pair L = 1048");
+    CHECK(!sort_in_line_pair(65536, (int64_t)85296 * 1048, epilogue), "pair, large table");
+  }
+}
+
 int main() {
   check_few_positions();
+  check_sorts_in_line();
   // the sort divides slot numbers by max_active (K) and positions by the
   // position-chunk rows (ceil(B / 2) or B); cover every K the ABI allows up to
   // 4096, the workloads' batches and chunk sizes, and powers of two
