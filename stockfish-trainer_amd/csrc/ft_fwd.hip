@@ -1418,7 +1418,7 @@ int fwd_f32(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int
   // flight.  Their lists end on whole 16-row steps; where that does not fit the
   // LDS lists (K from 4081, of the 4092 that do) the general mapping stays.
   const int kpad16 = (K + 15) / 16 * 16;
-  const bool few = vec && few_positions(B, K, cols) && index_lds_bytes(kWave, kpad16) <= kMaxIndexLds;
+  const bool few = vec && few_positions(B, K, cols, m.G, m.cpl) && index_lds_bytes(kWave, kpad16) <= kMaxIndexLds;
   if (few) m = Mapping{kWave, 1, (int)ceil_div(cols, (int64_t)kWave)};
   const int ppb = kWavesPerBlock * (kWave / m.G);
   const dim3 grid((unsigned)ceil_div(B, ppb), (unsigned)m.slabs);

@@ -55,22 +55,27 @@ struct FastDiv {
 // ---- the row gather's mapping of few positions ----
 // Whether B positions of `cols` 16-byte row chunks and K slots are gathered by a
 // wave per position and 64 chunks, 16 rows in flight, instead of the general
-// mapping (as many positions per wave as its rows are narrow, 4 rows in flight).
-// A position's rows are one chain of memory round trips, so the few-position
-// mapping wins while the launch is latency and loses once the rows' bytes, or
-// for narrow rows the waves themselves, are what takes the time.  General /
-// few-position, us (N = 23 232, K = 32; N = 85 296, K = 160 likewise by L, B):
-//   K = 32:  L = 32: 1024 6.4 / 4.8, 2048 6.2 / 5.5, 2560 6.2 / 6.5, 8192 6.2 / 11.6
-//            L = 256: 1024 7.7 / 6.3, 2048 9.7 / 9.2, 4096 14.4 / 15.2
-//            L = 520: 1024 15.0 / 11.3, 2048 19.3 / 19.5, 3072 25.4 / 27.2
-//            L = 1048: 256 13.7 / 7.6, 1024 19.8 / 18.7, 2048 32.9 / 33.6
-//   K = 160: L = 64: 3072 28.9 / 20.3, 8192 33.6 / 43.5;  L = 256: 1536 31.0 / 29.3, 2560 43.6 / 45.4
-//            L = 520: 1024 56 / 44, 1536 63 / 67;  L = 1048: 512 64 / 46, 1024 82 / 86
-SFT_HD inline bool few_positions(int64_t B, int K, int64_t cols) {
+// mapping (G lanes a position with cpl chunks each, 4 rows in flight).  A
+// position's rows are one chain of memory round trips, so the few-position
+// mapping wins while the launch is latency, the longer the more chunks the
+// general mapping's lanes take in turn, and loses once its waves or the rows'
+// bytes are what takes the time.  General / few-position, us:
+//   N = 23 232, K = 32: L = 40 (G = 16, cpl = 1) 2048 6 / 5, 3072 6 / 7, 8192 7 / 11;  L = 136 (8, 5) 2048 14 / 6,
+//   8192 17 / 16;  L = 168 (16, 3) 4096 14 / 11, 8192 17 / 19;  L = 248 (64, 1) 2048 10 / 9, 4096 15 / 16;
+//   L = 264 (16, 5) 2048 15 / 11, 4096 18 / 20;  L = 520 (32, 5) 1024 15 / 11, 2048 19 / 19, 4096 31 / 34;
+//   L = 904 (64, 4) 1024 17 / 17, 2048 28 / 34;  L = 1048 (64, 5) 256 14 / 8, 1536 26 / 26, 2048 33 / 34
+//   N = 85 296, K = 160: L = 56 3072 28 / 20, 6144 30 / 35;  L = 136 6144 67 / 63, 8192 77 / 81;  L = 168 4096 53 / 50,
+//   6144 73 / 75;  L = 248 2048 37 / 36, 3072 51 / 54;  L = 264 1536 54 / 35, 3072 64 / 67;  L = 392 512 32 / 20,
+//   1536 45 / 47;  L = 520 1024 52 / 43, 1536 63 / 67;  L = 1048 512 61 / 46, 1024 80 / 85;  L = 2048 512 105 / 77
+SFT_HD inline bool few_positions(int64_t B, int K, int64_t cols, int G, int cpl) {
   if (cols > 1 << 21) return false;  // a launch's column slabs stay below 2^16
-  if (K <= 32) return B <= 2048;
-  const int64_t most = (1 << 17) / cols;
-  return B <= (most < 768 ? 768 : most > 3072 ? 3072 : most);
+  const int64_t slabs = ceil_div(cols, 64);
+  if (slabs > 1) {  // the waves times their slots, and the batch
+    const int64_t halves = cpl > 4 ? 2 * (cpl - 3) : G < 64 ? 3 : 2;
+    return B <= (halves * 5 << 15) / (K * slabs) && B <= (cpl > 4 || G < 64 ? 2048 : 1536);
+  }
+  if (cpl == 1) return B <= (K > 64 && cols <= 16 ? 4096 : K > 32 && cols <= 32 ? 3072 : 2048);
+  return B <= (G > 8 ? 4096 : K <= 32 && cpl > 4 ? 8192 : 6144);
 }
 
 // ---- which sorts run on the caller's stream ----

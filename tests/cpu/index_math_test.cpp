@@ -195,23 +195,35 @@ static void check_chunk0_buckets(int64_t N, int nchunks, int sb) {
         (long long)(N >> sb));
 }
 
-// The row gather's few-position mapping, on both sides of its line: rows of one
-// 64-lane slab and of several, K up to 32 and above (16-byte chunks per row).
+// The row gather's few-position mapping, on both sides of its lines: rows of one
+// 64-chunk slab and of several, by the general mapping's lanes and chunks per
+// lane (choose_mapping's for these columns).
 static void check_few_positions() {
   struct Case {
     int64_t B;
     int K;
     int64_t cols;
+    int G, cpl;
     bool few;
   };
-  for (const Case &c : {Case{1, 32, 8, true}, Case{2048, 32, 8, true}, Case{2049, 32, 8, false},
-                        Case{8192, 32, 8, false}, Case{8192, 32, 32, false}, Case{4096, 32, 130, false},
-                        Case{256, 32, 262, true}, Case{2048, 32, 512, true}, Case{3072, 160, 16, true},
-                        Case{4097, 160, 16, false}, Case{8192, 160, 32, false}, Case{2048, 160, 64, true},
-                        Case{2560, 160, 64, false}, Case{1008, 160, 130, true}, Case{1536, 160, 130, false},
-                        Case{768, 160, 262, true}, Case{1024, 160, 262, false}, Case{512, 160, 512, true},
-                        Case{256, 4080, 1 << 20, true}, Case{1, 8, (1 << 21) + 1, false}})
-    CHECK(few_positions(c.B, c.K, c.cols) == c.few, "B=%lld K=%d cols=%lld", (long long)c.B, c.K, (long long)c.cols);
+  for (const Case &c : {
+           // one slab: chunks per lane 1, 3 and 5
+           Case{1, 32, 8, 8, 1, true}, Case{2048, 32, 8, 8, 1, true}, Case{2049, 32, 8, 8, 1, false},
+           Case{4096, 160, 14, 16, 1, true}, Case{4097, 160, 14, 16, 1, false}, Case{3072, 160, 30, 32, 1, true},
+           Case{3073, 64, 14, 16, 1, false}, Case{6144, 32, 18, 8, 3, true}, Case{6145, 32, 18, 8, 3, false}, Case{2048, 160, 62, 64, 1, true},
+           Case{2049, 160, 62, 64, 1, false}, Case{4096, 32, 42, 16, 3, true}, Case{4097, 160, 42, 16, 3, false},
+           Case{8192, 32, 34, 8, 5, true}, Case{8193, 32, 34, 8, 5, false}, Case{6144, 160, 34, 8, 5, true},
+           Case{6145, 160, 34, 8, 5, false},
+           // several
+           Case{2048, 32, 66, 16, 5, true}, Case{2049, 32, 66, 16, 5, false}, Case{1536, 32, 226, 64, 4, true},
+           Case{1537, 32, 226, 64, 4, false}, Case{256, 32, 262, 64, 5, true}, Case{2048, 32, 262, 64, 5, true},
+           Case{1024, 160, 130, 32, 5, true}, Case{1536, 160, 130, 32, 5, false}, Case{512, 160, 262, 64, 5, true},
+           Case{1024, 160, 262, 64, 5, false}, Case{1024, 160, 98, 64, 2, true}, Case{1025, 160, 98, 64, 2, false}, Case{1536, 160, 74, 32, 3, true},
+           Case{1537, 160, 74, 32, 3, false}, Case{2048, 32, 74, 32, 3, true}, Case{512, 160, 226, 64, 4, true},
+           Case{1280, 160, 512, 64, 8, true}, Case{1281, 160, 512, 64, 8, false},
+           Case{1, 8, (1 << 21) + 1, 64, 8, false}})
+    CHECK(few_positions(c.B, c.K, c.cols, c.G, c.cpl) == c.few, "B=%lld K=%d cols=%lld G=%d cpl=%d", (long long)c.B, c.K,
+          (long long)c.cols, c.G, c.cpl);
 }
 
 // Which sorts run in line, on both sides of each line: positions, slots per

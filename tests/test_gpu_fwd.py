@@ -62,10 +62,11 @@ def test_fwd_tiles_at_every_batch(seed, B, N, K, L, lo, hi, sort):
     assert np.array_equal(host(out), ft_oracle.fwd_f32(idx, W, b))
 
 
-# the row gather's mapping by batch: a wave per position and 64 chunks of it (K <= 32: up to 2048 positions;
-# K = 33: up to 2^17 / (L / 4) within 768 .. 3072), beyond that positions by the row's width
-@pytest.mark.parametrize("B,N,K,L", [(2048, 300, 3, 256), (2049, 300, 3, 256), (2047, 64, 17, 516),
-                                     (1008, 64, 33, 520), (1009, 64, 33, 520), (3072, 64, 33, 32), (3073, 64, 33, 32),
+# the row gather's mapping by batch: a wave per position and 64 chunks of it, beyond that positions by the row's
+# width; lines at one and at several 64-chunk slabs
+@pytest.mark.parametrize("B,N,K,L", [(2048, 300, 3, 32), (2049, 300, 3, 32), (8192, 64, 17, 136), (8193, 64, 17, 136),
+                                     (4096, 64, 33, 168), (4097, 64, 33, 168), (2048, 64, 17, 264), (2049, 64, 17, 264),
+                                     (1536, 64, 33, 392), (1537, 64, 33, 392),
                                      (1, 40, 1, 4), (8192, 300, 3, 256), (8193, 300, 3, 256), (4096, 64, 17, 512),
                                      (4097, 64, 17, 516), (33, 5000, 160, 1048), (2731, 90, 16, 1500)])
 def test_fwd_rows_few_positions(B, N, K, L):
