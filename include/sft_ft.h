@@ -82,8 +82,9 @@ int sft_ft_fwd_f32(const int32_t *idx, int64_t batch, int32_t max_active, const 
                    void *stream);
 
 /*
- * Bytes of device workspace sft_ft_fwd_f32_ex uses for these sizes and flags
- * (0 when the shape runs the row gather).  Host-only computation.
+ * Bytes of device workspace sft_ft_fwd_f32_ex and sft_ft_fwd_f32_prep use at most
+ * for these sizes and flags (0 when both run the row gather).  Host-only
+ * computation.
  * No reference counterpart (the reference kernel takes no workspace).
  */
 int sft_ft_fwd_f32_workspace_size(int64_t batch, int32_t max_active, int64_t num_inputs,

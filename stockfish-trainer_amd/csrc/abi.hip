@@ -17,7 +17,7 @@ int fwd_i16(const int32_t *idx, int64_t B, int K, const int16_t *W, int64_t N, i
 int quantize_i16(const float *x, int64_t n, float scale, int16_t *out, hipStream_t s);
 size_t fwd_tiled_workspace(int64_t B, int K, int64_t N, int L);
 bool fwd_tiled_supported(int64_t N, int L, const void *W, const void *bias, const void *out);
-bool fwd_tiled_pays(int64_t B, int K, int64_t N, int L);
+bool fwd_tiled_pays(int64_t B, int K, int64_t N, int L, bool beside_sort);
 int fwd_f32_tiled(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int L, const float *bias, float *out,
                   void *ws, size_t ws_bytes, hipStream_t s);
 int bwd_workspace(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *bytes);
@@ -43,6 +43,7 @@ int bwd_prep_bytes(int64_t B, int K, int64_t N, int L, uint32_t flags, size_t *b
 int bwd_prepare(const int32_t *idx, int64_t B, int K, int64_t N, int L, uint32_t flags, void *prep,
                 size_t prep_bytes, hipStream_t s);
 bool fwd_sort_in_line(int64_t B, int K, int64_t N, int L);
+bool fwd_sort_beside(int64_t B, int K, int64_t N, int L);
 size_t index_lds_bytes(int G, int K);
 int fwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, const FoldSrc &src, int64_t N, int L,
                  const float *bias, float *out0, float *out1, void *ws, size_t ws_bytes, hipStream_t s);
@@ -289,9 +290,10 @@ bool bad_sizes(int64_t B, int32_t K, int64_t N, int32_t L, std::string &why) {
 bool bad_fwd_flags(uint32_t flags) {
   return (flags & ~(SFT_FWD_ROWS | SFT_FWD_TILES)) || flags == (SFT_FWD_ROWS | SFT_FWD_TILES);
 }
-// Whether the flags, or without any the sizes, ask for the tiled gather.
-bool fwd_tiles(int64_t B, int32_t K, int64_t N, int32_t L, uint32_t flags) {
-  return (flags & SFT_FWD_TILES) || (!(flags & SFT_FWD_ROWS) && fwd_tiled_pays(B, K, N, L));
+// Whether the flags, or without any the sizes, ask for the tiled gather
+// (beside_sort: of a forward that sorts on the side stream).
+bool fwd_tiles(int64_t B, int32_t K, int64_t N, int32_t L, uint32_t flags, bool beside_sort) {
+  return (flags & SFT_FWD_TILES) || (!(flags & SFT_FWD_ROWS) && fwd_tiled_pays(B, K, N, L, beside_sort));
 }
 
 }  // namespace
@@ -341,7 +343,9 @@ int sft_ft_fwd_f32_workspace_size(int64_t batch, int32_t max_active, int64_t num
   if (bad_sizes(batch, max_active, num_inputs, output_size, why))
     return fail(SFT_EINVAL, "sft_ft_fwd_f32_workspace_size: " + why);
   if (bad_fwd_flags(flags)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_workspace_size: unknown flags");
-  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
+  // the forward that sorts beside its gather takes the tiles at smaller batches: the size covers it
+  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags,
+                               fwd_sort_beside(batch, max_active, num_inputs, output_size)) &&
                      fwd_tiled_supported(num_inputs, output_size, nullptr, nullptr, nullptr);
   *bytes = tiled ? fwd_tiled_workspace(batch, max_active, num_inputs, output_size) : 0;
   return SFT_OK;
@@ -356,7 +360,7 @@ int sft_ft_fwd_f32_ex(const int32_t *idx, int64_t batch, int32_t max_active, con
   if (!weight || !bias || (batch > 0 && (!idx || !out))) return fail(SFT_EINVAL, "sft_ft_fwd_f32_ex: null pointer");
   if (bad_fwd_flags(flags)) return fail(SFT_EINVAL, "sft_ft_fwd_f32_ex: unknown flags");
   if (batch == 0) return SFT_OK;
-  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
+  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags, false) &&
                      fwd_tiled_supported(num_inputs, output_size, weight, bias, out) &&
                      workspace != nullptr &&
                      workspace_bytes >= fwd_tiled_workspace(batch, max_active, num_inputs, output_size);
@@ -421,7 +425,8 @@ int sft_ft_fwd_f32_prep(const int32_t *idx, int64_t batch, int32_t max_active, c
   if (!forked) side_join.release();
   if ((rc = bwd_prepare(idx, batch, max_active, num_inputs, output_size, bwd_flags, prep, prep_bytes, side)) != SFT_OK)
     return rc;
-  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags) &&
+  const bool tiled = fwd_tiles(batch, max_active, num_inputs, output_size, flags,
+                               fwd_sort_beside(batch, max_active, num_inputs, output_size)) &&
                      fwd_tiled_supported(num_inputs, output_size, weight, bias, out) &&
                      workspace != nullptr &&
                      workspace_bytes >= fwd_tiled_workspace(batch, max_active, num_inputs, output_size);

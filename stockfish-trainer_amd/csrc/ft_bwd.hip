@@ -1648,6 +1648,10 @@ static bool narrow_rows(int K, int L) { return (int64_t)K * SFT_BWD_SPLIT_K_PER_
 bool fwd_sort_in_line(int64_t B, int K, int64_t N, int L) {
   return sort_in_line_fwd(B * K, K, L, narrow_rows(K, L), table_parts(N) == 1);
 }
+// Whether a forward that prepares the backward's sort does so on the side stream.
+bool fwd_sort_beside(int64_t B, int K, int64_t N, int L) {
+  return prep_pays(B, K, L, SFT_BWD_OVERWRITE) && !fwd_sort_in_line(B, K, N, L);
+}
 static bool bwd_sort_in_line(int64_t B, int K, int64_t N, int L, bool prepared) {
   return sort_in_line_bwd(B * K, K, narrow_rows(K, L), prepared, table_parts(N) == 1);
 }

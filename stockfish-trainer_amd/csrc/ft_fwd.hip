@@ -1577,23 +1577,33 @@ bool fwd_tiled_supported(int64_t N, int L, const void *W, const void *bias, cons
          (uintptr_t)W % 16 == 0 && (uintptr_t)bias % 16 == 0 && (uintptr_t)out % 16 == 0;
 }
 
-// Whether the tiled gather of a shape it supports is the faster one.  It copies
-// the whole table first (2 T bytes at 5 TB/s, then the rank lists: about 6 us,
-// 26 us for lists of more than 32 slots, and 12 us a further table part); the row gather reads only the rows
-// it sums, but from beyond L2, so per byte it loses `slower`: the bytes of rows
-// (three quarters of the slots active) at which the two meet, per us of that
-// first cost, fall as the table outgrows the 4 MB L2s.  Tiled / row gather, us,
-// around the line (N, K, L, B):
-//   23 232, 32, 1048: 3072 55 / 47, 4096 59 / 62;  520: 3072 32 / 28, 4096 34 / 36
-//   8192, 32, 1048: 1536 27 / 23, 2048 29 / 31;  264: 12 288 29 / 27, 16 384 32 / 35
-//   517, 32, 1048: 8192 40 / 39, 16 384 65 / 68
-//   85 296, 160, 1048: 6144 382 / 372, 8192 428 / 488;  136: 12 288 111 / 108
-// and far from it: 23 232, 32, 1048, B = 256 42 / 5.9, B = 65 536 285 / 930.
-bool fwd_tiled_pays(int64_t B, int K, int64_t N, int L) {
-  const double table_mb = 4e-6 * N * L, rows_mb = 3e-6 * B * K * L;
-  const int parts = table_parts(N);
-  const double slower = parts > 1 ? 13 : table_mb > 20 ? 9 : table_mb > 14 ? 12 : table_mb > 4.5 ? 35 : 100;
-  return rows_mb > slower * (0.4 * table_mb + (K <= kRankStageMaxPad ? 6 : 26) + 12 * (parts - 1));
+// Whether the tiled gather of a shape it supports is the faster one: the time of
+// each in us, with three quarters of the slots active.
+//   rows: each row from L2 (45 us a GB) or, for what of the table lies beyond it,
+//     from the memory side (147 us a GB); a row's ends cost it 16 bytes more.
+//   tiles: the table's copy (0.27 us a MB), the rank lists (4 us a million slots,
+//     28 us more for rows of more than 32), the rows from L2 (34 us a GB), and for
+//     each further table part its launch and carried sums.
+// beside_sort: a sort runs on the side stream meanwhile; the copy and the tiled
+// gather hide it, the row gather leaves 20 us of it a million slots.
+// Continuous in every size, so that no step of the rule is far from the point
+// where the two meet.  Tiled / row gather, us, on both sides of it (N, K, L, B):
+//   1100, 32, 1048: 4000 28 / 24, 8000 42 / 43;  3200: 2000 24 / 21, 3000 27 / 30;  4200: 1500 22 / 20, 2500 26 / 30
+//   5000, 32, 1048: 1500 22 / 21, 2500 27 / 32;  23 232: 3000 55 / 47, 4000 59 / 61;  30 000 (2 parts): 6000 105 / 94,
+//   12 000 152 / 180;  8192, 32, 264: 12 000 30 / 26, 16 000 33 / 35;  23 232, 32, 136: 16 000 28 / 23, 32 000 37 / 46
+//   23 232, 160, 520: 2000 82 / 65, 3000 91 / 98;  85 296: 5000 204 / 180, 8000 244 / 283
+//   85 296, 160, 1048: 4000 355 / 289, 6000 407 / 441;  136: 10 000 115 / 113, 16 000 139 / 142
+// with a sort beside, both gathers of an evaluation: 85 296, 160, 136: 8192 225 / 213, 10 000 246 / 266;
+//   264: 6000 289 / 269, 9000 340 / 382.
+// Far from it: 23 232, 32, 1048, B = 256 42 / 7.6, B = 65 536 285 / 930.
+bool fwd_tiled_pays(int64_t B, int K, int64_t N, int L, bool beside_sort) {
+  const double table_mb = 4e-6 * N * L, mslots = 1e-6 * B * K, rows_mb = 3.0 * mslots * L;
+  const int more_parts = table_parts(N) - 1;
+  const double in_l2 = std::min(1.0, 7.5 / table_mb);
+  const double rows = 4 + (rows_mb + 12 * mslots) * (0.147 - 0.102 * in_l2) + (beside_sort ? 20 * mslots : 0);
+  const double tiles = 12 + (K > kRankStageMaxPad ? 28 : 0) + 0.27 * table_mb + 4 * mslots +
+                       rows_mb * (0.034 + 0.004 * more_parts) + more_parts * (14 + 0.09 * table_mb);
+  return tiles < rows;
 }
 
 int fwd_f32_tiled(const int32_t *idx, int64_t B, int K, const float *W, int64_t N, int L, const float *bias, float *out,

@@ -254,6 +254,45 @@ def rank_lists_bytes(B, K):
     return _a256(bp * kpad * 4) + 2 * _a256(bp * 4) + 2 * _a256(bp * 16)
 
 
+def _fwd_tiles(B, K, N, L):
+    """Whether the forward takes the tiled gather (its workspace holds the tiles)."""
+    n = ctypes.c_size_t()
+    assert _native.lib().sft_ft_fwd_f32_workspace_size(B, K, N, L, _native.SFT_FWD_AUTO, ctypes.byref(n)) == 0
+    return n.value > 0
+
+
+def _first_tiled_batch(K, N, L):
+    lo, hi = 0, 1 << 20  # rows at lo, tiles at hi
+    assert _fwd_tiles(hi, K, N, L)
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (lo, mid) if _fwd_tiles(mid, K, N, L) else (mid, hi)
+    return hi
+
+
+@pytest.mark.parametrize("K,N,L,rows,tiles", [
+    (32, 1100, 1048, 4000, 12000), (32, 3200, 1048, 2000, 3000), (32, 4200, 1048, 1500, 2500), (32, 5000, 1048, 1500, 2500),
+    (32, 23232, 1048, 3000, 4000), (32, 30000, 1048, 6000, 12000), (32, 23232, 520, 3000, 6000),
+    (32, 23232, 136, 16000, 32000), (160, 23232, 520, 2000, 3000), (160, 85296, 1048, 4000, 6000),
+    (160, 85296, 520, 4096, 8000), (160, 85296, 264, 6000, 9000), (160, 85296, 136, 8192, 16000)])
+def test_forward_route_on_both_sides_of_its_line(K, N, L, rows, tiles):
+    """Batches at which the row gather, and the tiled one, measured faster."""
+    assert rows < _first_tiled_batch(K, N, L) <= tiles
+
+
+@pytest.mark.parametrize("K,L,sizes", [(32, 1048, (400, 28000)), (32, 264, (1500, 28000)), (160, 520, (2000, 28000)),
+                                       (160, 1048, (60000, 85000))])
+def test_forward_route_has_no_step_in_the_table(K, L, sizes):
+    """The line moves with the table's rows without a jump: a table 2% larger moves it
+    by less than a quarter (within one count of table parts)."""
+    prev, n = None, sizes[0]
+    while n < sizes[1]:
+        b = _first_tiled_batch(K, n, L)
+        if prev is not None and not (57344 <= n < 58600):
+            assert 0.8 < b / prev < 1.25, (n, prev, b)
+        prev, n = b, int(n * 1.02) + 1
+
+
 @pytest.mark.parametrize("N", [500, 3000, 24576, 140000])
 @pytest.mark.parametrize("K", [4, 32, 160])
 @pytest.mark.parametrize("L", [264, 1048])
