@@ -317,15 +317,18 @@ def test_prepared_bwd_reads_the_buffer_only(B, L):
 
 
 @pytest.mark.parametrize("N", [1023, 1024, 1025, 1152])
-def test_prepared_bwd_chunk0_buckets_edge(N):
-    """The split prepared sort's buckets run in two launches, those holding
-    every key of position chunk 0 and the first key of chunk 1 (key N, whose
-    segment start ends chunk 0's last segment) first.  Feature counts at and
-    around a multiple of the 128-key bucket (N = 1024, 1152: key N opens a
-    bucket of its own) keep the weight grad bit-exact (B = 40000: two position
-    chunks; L = 136: K >= L / 5)."""
-    announce(f"prepared bwd, chunk-0 buckets N={N}")
-    B, K, L = 40000, 32, 136
+@pytest.mark.parametrize("B", [40000, 98400])
+def test_prepared_bwd_chunk0_buckets_edge(B, N):
+    """The split prepared sort's buckets (L = 136: K >= L / 5) over two position
+    chunks.  On the side stream (B = 98400: more than 3 x 2^20 slots) they run in
+    two launches, those holding every key of position chunk 0 and the first key
+    of chunk 1 (key N, whose segment start ends chunk 0's last segment) first,
+    and chunk 0's gather waits for that launch only; in line (B = 40000) in one.
+    Feature counts at and around a multiple of the 128-key bucket (N = 1024, 1152:
+    key N opens a bucket of its own) keep the weight grad bit-exact.
+    (test_gpu_graph.py captures the two launches at B = 40000.)"""
+    announce(f"prepared bwd, chunk-0 buckets B={B} N={N}")
+    K, L = 32, 136
     idx, W, b, G = case(40 + N % 7, B, N, K, L, 0, 32, True)
     _, i, prep = _prepare(idx, N, L)
     dW, db = _prepared_bwd(i, G, N, prep)

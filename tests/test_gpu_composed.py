@@ -50,11 +50,15 @@ SHAPES = [
     (9, 5003, 32, 1048, 0, 32, [(24576, 768)]),  # one launch for both perspectives, two tiles a workgroup
     (10, 16384, 8, 264, 0, 8, [(3072, 96), (700, 0)]),  # its largest batch, one tile a workgroup, skewed
     (11, 16385, 8, 264, 0, 8, [(3072, 96), (700, 0)]),  # a launch per perspective, one position chunk, skewed
+    # the largest table of the one-launch sort (2 N keys of 18 bits), and one past it: a launch per perspective,
+    # two tiles a workgroup, the second adding onto the first's rows; skewed
+    (12, 3000, 32, 256, 0, 32, [(131072, 0)]),
+    (13, 3000, 32, 256, 0, 32, [(131000, 0), (80, 0)]),
     (6, 6000, 32, 520, 16, 32, [(40, 8), (24, 0)]),  # 64 rows, one position chunk: every segment long
     (7, 40000, 32, 520, 16, 32, [(40, 8), (24, 0)]),  # two position chunks: long segments in both
     (8, 40000, 32, 520, 16, 32, [(3072, 96), (700, 0)]),  # two chunks, Zipf-skewed: hot and short segments
 ]
-ZIPF = {8: 1.0, 9: 0.7, 10: 1.0, 11: 1.0}  # seeds whose rows draw features with skewed frequencies
+ZIPF = {8: 1.0, 9: 0.7, 10: 1.0, 11: 1.0, 12: 1.0, 13: 1.0}  # seeds whose rows draw features with skewed frequencies
 
 
 def _indices(g, seed, B, N, K, lo, hi, sort):

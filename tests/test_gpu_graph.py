@@ -8,7 +8,8 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_helpers import DEV, announce, case, dev
+from gpu_helpers import DEV, announce, case, dev, host
+from oracle import ft_oracle
 from src.model.modules.feature_transformer import SparseLinearFunction
 from src.model.modules.features import get_feature_cls
 from src.model.transform_inputs import transform_inputs
@@ -85,6 +86,29 @@ def test_graph_skewed_segments(L):
         return [ow, ob, Wt.grad, bt.grad]
 
     _capture_and_compare(step, 4)
+
+
+@pytest.mark.parametrize("N", [1023, 1024, 1025, 1152])
+def test_graph_split_prepared_buckets(N):
+    """A captured narrow step of two position chunks forks its sorts, so the
+    prepared backward's buckets run in two launches on the side stream: chunk 0's
+    gather waits for the first, chunk 1's for both.  Feature counts at and
+    around a multiple of the 128-key bucket; every replay bit-exact."""
+    announce(f"graph: split prepared buckets N={N}")
+    B, K, L = 40000, 32, 136
+    idx, W, b, G = case(60 + N % 7, B, N, K, L, 0, 32, True)
+    i, g = dev(idx), dev(G)
+    Wt, bt = dev(W).requires_grad_(True), dev(b).requires_grad_(True)
+
+    def step():
+        Wt.grad = None
+        bt.grad = None
+        out = SparseLinearFunction.apply(i, Wt, bt)
+        out.backward(g)
+        return [out, Wt.grad, bt.grad]
+
+    assert np.array_equal(host(step()[1]), ft_oracle.bwd_f32(idx, G, N)[0])
+    _capture_and_compare(step, 3)
 
 
 def test_graph_fused_transform():
