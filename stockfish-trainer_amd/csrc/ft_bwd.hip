@@ -422,7 +422,7 @@ __global__ __launch_bounds__(kBlock) void gather_rows_kernel(const int32_t *__re
 // buffer (tmp_row), half 1 loads that value and keeps adding.  Either way a feature's sum is acc = 0,
 // acc += grad[b] over its positions ascending: the reference order
 // (FT/kernel.py:122, 178-181), bit for bit.  A lane group of 8 lanes x 16 B
-// owns one feature's tile row; tiles go to XCDs whole (tile_sched_item), so an
+// owns one feature's tile row; tiles go to XCDs whole (TileSched), so an
 // XCD reads one tile-half of Gt at a time: 32768 x 128 B = 4 MB, its L2.
 // The summed tile rows are written once per launch and read back, if at all,
 // by the next launch.  When a tile-half of the grad tiles takes half of an

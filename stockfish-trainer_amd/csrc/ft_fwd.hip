@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void fwd_i16_kernel(const int32_t *__restri
 // The table is first re-laid out as column tiles: tile t holds columns
 // [32t, 32t + 32) of every row, 128 bytes per row, rows contiguous, so one
 // tile is N * 128 B (2.97 MB for N = 23 232) and fits one XCD's 4 MB L2.
-// The gather then runs tile by tile on each XCD (tile_sched_item), lane
+// The gather then runs tile by tile on each XCD (TileSched), lane
 // groups of 8 lanes x 16 B covering one tile row per position, so every
 // table read after the first touch of a tile is an L2 hit.
 //

@@ -734,14 +734,14 @@ int slot_sort_buckets_high(const int32_t *idx, int64_t M, int K, int64_t N, int 
   const unsigned nkeys = (unsigned)((int64_t)nchunks * N);
   const SlotKey sk{idx, idx1 ? idx1 : idx, idx1 ? M / 2 : M, (unsigned)N, FastDiv((uint32_t)K),
                    FastDiv((uint32_t)chunk_rows), nkeys};
-#define SFT_HIGH_PASS(RB)                                                                                          \
-  rc = sort_big(M, RB) ? run_high_pass<RB, kBigItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,      \
-                                                  clear, nclear, s)                                               \
-                   : run_high_pass<RB, kSmallItems>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles,    \
-                                                    clear, nclear, s)
-  if (bb.rb == 8) SFT_HIGH_PASS(8);
-  else if (bb.rb == 9) SFT_HIGH_PASS(9);
-  else SFT_HIGH_PASS(10);
+#define SFT_HIGH_PASS(RB, IT) \
+  rc = run_high_pass<RB, IT>(sk, M, bb.sb, bb.k1, bb.v1, bb.hist, bb.totals, bb.ntiles, clear, nclear, s)
+  const bool big = sort_big(M, bb.rb);  // 10-bit digits always
+  if (bb.rb == 8 && big) SFT_HIGH_PASS(8, kBigItems);
+  else if (bb.rb == 8) SFT_HIGH_PASS(8, kSmallItems);
+  else if (bb.rb == 9 && big) SFT_HIGH_PASS(9, kBigItems);
+  else if (bb.rb == 9) SFT_HIGH_PASS(9, kSmallItems);
+  else SFT_HIGH_PASS(10, kBigItems);
 #undef SFT_HIGH_PASS
   return rc;
 }

@@ -189,9 +189,6 @@ struct TileSched {
     return TileItem{(int)(kXcds * full + t), (int)c};
   }
 };
-SFT_HD inline TileItem tile_sched_item(int64_t bid, int ntiles, int nchunks) {
-  return TileSched(ntiles, nchunks).item((uint32_t)bid);
-}
 
 // ---- column maps of the 32-column tiles ----
 // Tile t, lane q (one 16-byte chunk of 4 columns) of a tile row holds chunk

@@ -52,10 +52,11 @@ static void check_fastdiv(uint32_t d) {
 // whole residue classes of the chunk index mod 8.
 static void check_schedule(int ntiles, int nchunks) {
   const int64_t blocks = tile_sched_items_per_xcd(ntiles, nchunks) * kXcds;
+  const TileSched sched(ntiles, nchunks);
   std::vector<int> seen((size_t)ntiles * nchunks, 0);
   std::vector<std::vector<int>> xcd_tiles(kXcds);
   for (int64_t b = 0; b < blocks; ++b) {
-    const TileItem it = tile_sched_item(b, ntiles, nchunks);
+    const TileItem it = sched.item((uint32_t)b);
     if (it.tile >= ntiles) {
       CHECK(it.tile == ntiles, "ntiles=%d nchunks=%d b=%lld tile=%d", ntiles, nchunks, (long long)b, it.tile);
       continue;
@@ -81,7 +82,7 @@ static void check_schedule(int ntiles, int nchunks) {
   if (rem) {
     std::vector<std::vector<std::pair<int, int>>> left(kXcds);  // (tile, chunk) in launch order
     for (int64_t b = 0; b < blocks; ++b) {
-      const TileItem it = tile_sched_item(b, ntiles, nchunks);
+      const TileItem it = sched.item((uint32_t)b);
       if (it.tile >= full * kXcds && it.tile < ntiles) left[b % kXcds].push_back({it.tile, it.chunk});
     }
     const int64_t lo = (int64_t)rem * (nchunks / kXcds), hi = (int64_t)rem * ((nchunks + kXcds - 1) / kXcds);
