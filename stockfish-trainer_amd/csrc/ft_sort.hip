@@ -27,8 +27,9 @@ namespace {
 // 16 above.  A small sort is a chain of latencies in a few workgroups: with
 // 4096-slot tiles 320 K slots filled 79 of them (downsweep 13.0 -> 7.8 us).  A
 // large one pays per tile, for its digit counts and the scans that walk them,
-// and shares the GPU: 2.1 M slots, both perspectives' steps with 4 / 8 / 16 per
-// thread, L = 136 387 / 369 / 366 us, L = 1048 1668 / 1645 / 1634 us.
+// and shares the GPU.  Both perspectives' steps with 16 / 4 per thread, K = 32,
+// N = 23 232, us: L = 1048: 2^18 slots 431 / 421, 2^19 559 / 561, 640 K 629 / 636, 2^20 869 / 883,
+// 2^21 1651 / 1674;  L = 136: 2^19 167 / 159, 2^20 231 / 230, 1.4 M 301 / 304, 2^21 369 / 390.
 // (The count buffer has 2^10 counts per 2048 slots, which 1024-slot tiles fill
 // with 9-bit digits; 10-bit ones keep the large tiles.)
 constexpr int64_t kSmallSlots = 1 << 19;
