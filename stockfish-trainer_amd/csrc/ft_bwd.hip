@@ -2014,10 +2014,10 @@ static int pair_sort_both(const int32_t *idx0, const int32_t *idx1, int64_t B, i
 // Both perspectives' slots in one sort on the side stream (key = perspective N +
 // feature, positions of perspective 1 from B on); joined by the caller when
 // *forked.
-static int pair_sort_once(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, int64_t N, int L, bool epilogue,
-                          char *sort_ws, int32_t *seg, SortedSlots &out, bool *forked, hipStream_t s) {
+static int pair_sort_once(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, int64_t N, int L, char *sort_ws,
+                          int32_t *seg, SortedSlots &out, bool *forked, hipStream_t s) {
   hipStream_t side;
-  int rc = fork_sort(s, sort_in_line_pair(B * K, N * L, epilogue), &side, forked);
+  int rc = fork_sort(s, sort_in_line_pair(B * K, N * L), &side, forked);
   if (rc != SFT_OK) return rc;
   SideJoinGuard side_join(s);
   if (!*forked) side_join.release();
@@ -2066,8 +2066,8 @@ int bwd_pair_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K, con
   if (lay.one_launch) {
     f32x4 *gt1 = reinterpret_cast<f32x4 *>(w + lay.gt1);
     bool forked;
-    if ((rc = pair_sort_once(idx0, idx1, B, K, N, L, false, w + lay.sort[0],
-                             reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], &forked, s)) != SFT_OK)
+    if ((rc = pair_sort_once(idx0, idx1, B, K, N, L, w + lay.sort[0], reinterpret_cast<int32_t *>(w + lay.seg[0]),
+                             ss[0], &forked, s)) != SFT_OK)
       return rc;
     SideJoinGuard side_join(s);
     if (!forked) side_join.release();
@@ -2172,7 +2172,7 @@ int bwd_transform_f32(const int32_t *idx0, const int32_t *idx1, int64_t B, int K
   e.P = L - L1;
   SortedSlots ss[2];  // sorted on the side stream while the epilogue runs
   bool forked = true;
-  int rc = lay.one_launch ? pair_sort_once(idx0, idx1, B, K, N, L, true, w + lay.sort[0],
+  int rc = lay.one_launch ? pair_sort_once(idx0, idx1, B, K, N, L, w + lay.sort[0],
                                            reinterpret_cast<int32_t *>(w + lay.seg[0]), ss[0], &forked, s)
                           : pair_sort_both(idx0, idx1, B, K, N, lay.nc, w, lay.sort, lay.seg, ss, s);
   if (rc != SFT_OK) return rc;

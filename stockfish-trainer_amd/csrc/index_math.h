@@ -92,15 +92,17 @@ SFT_HD inline bool few_positions(int64_t B, int K, int64_t cols, int G, int cpl)
 // it hides: for lists of more than 32 slots the line is on M L.
 //   K = 32, N = 23 232, L = 136: B = 16 384 173 / 159, 65 536 385 / 376, 100 000 548 / 537, 131 072
 //   741 / 725;  N = 85 296: 65 536 696 / 691, 131 072 1159 / 1169
-//   K = 64, N = 23 232, L = 264: 8192 235 / 238, 32 768 492 / 505, 65 536 898 / 921 (host-bound below
-//   24 000: 16 384 402 / 313);  K = 128, L = 520: 5000 378 / 394 (host-bound 408 / 386), 8000 468 / 484
+//   K = 64, N = 23 232, L = 264: 8192 235 / 238, 16 384 305 / 320 (host-bound 402 / 313), 32 768 492 / 505 (a step
+//   waited for by itself, on a slow host 707 / 589), 65 536 898 / 921;  K = 128, L = 520: 5000 378 / 394 (host-bound
+//   408 / 386), 8000 468 / 484 (by itself 663 / 564)
 //   K = 160, N = 85 296, L = 136: 8192 391 / 384, 10 000 444 / 453;  L = 520: 1000 348 / 343, 3000 601 / 617;
 //   L = 800: 1000 469 / 462, 3000 811 / 828
 // Wide rows (the whole sort in the forward): K = 64, N = 23 232, L = 1048: 1000 238 / 227, 2048 347 / 348;
-// K = 32, L = 264: 6000 170 / 164, 12 000 192 / 194;  K = 160, N = 85 296, L = 1048: 64 442 / 443, 409 502 / 514.
+// K = 32, L = 264: 6000 170 / 164, 12 000 192 / 194;  K = 160, N = 85 296, L = 1048: 409 502 / 514, but a step
+// waited for by itself 686 / 631.
 SFT_HD inline bool sort_in_line_fwd(int64_t M, int K, int L, bool narrow, bool one_part) {
-  if (!narrow) return M <= (one_part ? 1 << 16 : 1 << 14);
-  if (K > 32 && M * L > (one_part ? (int64_t)3 << 27 : (int64_t)3 << 26)) return false;
+  if (!narrow) return M <= 1 << 16;
+  if (K > 32 && M * L > (one_part ? (int64_t)5 << 27 : (int64_t)3 << 26)) return false;
   return M <= (one_part ? 3 << 20 : 1 << 21);
 }
 // The backward's: the buckets of a prepared sort, or (not prepared) the whole sort.
@@ -114,15 +116,13 @@ SFT_HD inline bool sort_in_line_bwd(int64_t M, int K, bool narrow, bool prepared
   if (!narrow) return M <= 1 << 16;
   return M <= (!prepared || (K <= 32 && !one_part) ? 1 << 21 : 3 << 20);
 }
-// Both perspectives' sort of a composed backward over a table of so many values,
-// M slots each; epilogue: beside the post-FT epilogue's backward, which hides
-// more of it.  Host-bound steps (small tables) gain 40 us in line, the others
-// lose:  composed, N = 24 576, L = 1048, B = 2048 213 / 214 (host-bound 297 / 252);  N = 85 296: 545 / 550;
-// epilogue, N = 24 576: L = 264 141 / 148 (host-bound 324 / 290), L = 1048 375 / 384 (host-bound 379 / 389);
-// N = 85 296: L = 264 247 / 262 (host-bound 348 / 303), L = 1048 703 / 719.
-SFT_HD inline bool sort_in_line_pair(int64_t M, int64_t table, bool epilogue) {
-  return M <= 1 << 16 && table <= (epilogue ? 24 : 48) * (int64_t)1000000;
-}
+// Both perspectives' sort of a composed or epilogue backward over a table of so
+// many values, M slots each.  Steps that the host bounds gain 40 us in line, and
+// from about 500 us of kernels on none is bound by it: forked / in line, B = 300,
+// composed, N = 24 576, L = 1048 297 / 252, N = 85 296: L = 648 390 / 335 (a faster host 327 / 324), L = 1048 447 / 453;
+// epilogue, N = 24 576: L = 264 325 / 285, L = 1048 350 / 349 (waited for by itself 561 / 537), N = 85 296: L = 264
+// 350 / 305, L = 648 439 / 415 (a faster host 393 / 412), L = 808 488 / 505 (alone 700 / 675), L = 1048 606 / 623.
+SFT_HD inline bool sort_in_line_pair(int64_t M, int64_t table) { return M <= 1 << 16 && table <= 80 * (int64_t)1000000; }
 
 // ---- XCD-aware tile schedule ----
 // MI355X runs a dispatch's workgroups round-robin over its 8 XCDs (workgroup i
