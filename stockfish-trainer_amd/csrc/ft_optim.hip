@@ -77,13 +77,29 @@ constexpr int kOptRowChunks = 8;  // 16-byte chunks per lane kept in registers (
 // 2-D tables, cols % 4 == 0 and cols <= 4 * 64 * kOptRowChunks: one wave per row,
 // the whole row of all five tensors loaded into registers before the norm's
 // reduction, so the loads of a row are all in flight together.  Bound by HBM
-// (20 bytes read, 12 written per element).  Plain loads and stores: non-temporal
-// ones are faster only where such updates follow each other (25 344 rows of 1048,
-// three sets of tensors in turn 173 -> 168 us) and slower with a step's other
-// traffic between them, as in training (a 1 GB copy between updates: 24 576 x 1048
-// 152 -> 159 us, 60 720 x 1048 391 -> 411), and for smaller tables even in turn
-// (24 576 x 264 42 -> 48).
-template <int NCH>
+// (20 bytes read, 12 written per element).
+// NT: non-temporal loads and stores, for tables whose five tensors together are
+// past the 256 MB MALL, which then only passes their lines on, up to 600 MB.
+// Below, a second update finds lines of the first in the MALL; far above,
+// non-temporal stores cost more than they save.  Plain / NT, us, four sets of tensors in turn (two):
+//   24 576 x 264 (130 MB) 42.3 / 41.2 (42.6 / 48.2);  8000 x 520 (83 MB) 24.8 / 27.1 (31.8 / 36.2)
+//   24 576 x 520 (256 MB) 80.3 / 77.4 (89.8 / 86.8);  16 000 x 1048 (335 MB) 104.7 / 101.2 (119.0 / 114.9)
+//   24 576 x 1048 (515 MB) 157.9 / 155.2 (171.8 / 167.9);  60 720 x 520 (631 MB) 189 / 190 (200 / 201)
+//   60 720 x 1048 (1273 MB) 392 / 402 (405 / 417)
+// Behind a step's forward and backward the line is nearly even (the step and its
+// update, 24 576 x 1048: 409 / 396 us at 2048 positions, 717 / 715 at 16 384,
+// 1792 / 1800 at 65 536); behind a 1 GB copy plain is faster (152 / 159).
+constexpr int64_t kOptNtBytes = 240ll * 1000000, kOptNtMaxBytes = 600ll * 1000000;
+template <bool NT>
+__device__ __forceinline__ f32x4 opt_load(const f32x4 *p) {
+  return NT ? __builtin_nontemporal_load(p) : *p;
+}
+template <bool NT>
+__device__ __forceinline__ void opt_store(f32x4 v, f32x4 *p) {
+  if (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+template <int NCH, bool NT>
 __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restrict__ p, const f32x4 *__restrict__ g,
                                                                  f32x4 *__restrict__ v, f32x4 *__restrict__ m,
                                                                  const f32x4 *__restrict__ mp, int64_t rows,
@@ -99,11 +115,11 @@ __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restri
   for (int j = 0; j < NCH; ++j) {
     const int c = lane + kWave * j;
     const bool ok = c < cols4;
-    pr[j] = ok ? p[base + c] : z;
-    gr[j] = ok ? g[base + c] : z;
-    vr[j] = ok ? v[base + c] : z;
-    mr[j] = ok ? m[base + c] : z;
-    mpr[j] = ok ? mp[base + c] : z;
+    pr[j] = ok ? opt_load<NT>(p + base + c) : z;
+    gr[j] = ok ? opt_load<NT>(g + base + c) : z;
+    vr[j] = ok ? opt_load<NT>(v + base + c) : z;
+    mr[j] = ok ? opt_load<NT>(m + base + c) : z;
+    mpr[j] = ok ? opt_load<NT>(mp + base + c) : z;
   }
   float sq = 0.f;
 #pragma unroll
@@ -123,9 +139,9 @@ __global__ __launch_bounds__(kBlock) void ranger_rows_vec_kernel(f32x4 *__restri
       vv[e] = ve;
       mv[e] = me;
     }
-    p[base + c] = pv;
-    v[base + c] = vv;
-    m[base + c] = mv;
+    opt_store<NT>(pv, p + base + c);
+    opt_store<NT>(vv, v + base + c);
+    opt_store<NT>(mv, m + base + c);
   }
 }
 
@@ -164,11 +180,13 @@ int ranger_update_f32(float *p, const float *grad, float *variance_ma, float *gm
   if (vec) {
     const int cols4 = (int)(cols / 4);
     const dim3 grid((unsigned)ceil_div(rows, kWavesPerBlock));
+    const int64_t bytes = 20 * rows * cols;
+    const bool nt = bytes >= kOptNtBytes && bytes <= kOptNtMaxBytes;
 #define SFT_RANGER_VEC(NCH)                                                                                     \
-  hipLaunchKernelGGL(ranger_rows_vec_kernel<NCH>, grid, dim3(kBlock), 0, s, reinterpret_cast<f32x4 *>(p),      \
-                     reinterpret_cast<const f32x4 *>(grad), reinterpret_cast<f32x4 *>(variance_ma),            \
-                     reinterpret_cast<f32x4 *>(gma_cur), reinterpret_cast<const f32x4 *>(gma_prev), rows, cols4, \
-                     scalars)
+  hipLaunchKernelGGL((nt ? ranger_rows_vec_kernel<NCH, true> : ranger_rows_vec_kernel<NCH, false>), grid,       \
+                     dim3(kBlock), 0, s, reinterpret_cast<f32x4 *>(p), reinterpret_cast<const f32x4 *>(grad),   \
+                     reinterpret_cast<f32x4 *>(variance_ma), reinterpret_cast<f32x4 *>(gma_cur),                \
+                     reinterpret_cast<const f32x4 *>(gma_prev), rows, cols4, scalars)
     if (cols4 <= 2 * kWave)
       SFT_RANGER_VEC(2);
     else if (cols4 <= 5 * kWave)

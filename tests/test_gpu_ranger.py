@@ -37,7 +37,9 @@ def _ulps(a, b):
     return np.abs(ai - bi)
 
 
-@pytest.mark.parametrize("shape", [(24576, 1048), (768, 1048), (1048,), (37, 13), (5, 2100), (300, 256), (1, 4)])
+@pytest.mark.parametrize("shape", [(24576, 1048), (768, 1048), (1048,), (37, 13), (5, 2100), (300, 256), (1, 4),
+                                   # both sides of the lines of the non-temporal accesses, 12 and 30 M elements
+                                   (46875, 256), (46874, 256), (6000, 2000), (15000, 2000), (15001, 2000)])
 def test_fused_update_matches_oracle(shape):
     announce(f"ranger22 update shape={shape}")
     p, g, v, m, mp, sc = _inputs(len(shape) * 100 + shape[0], shape)
