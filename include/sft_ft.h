@@ -132,8 +132,10 @@ int sft_ft_bwd_f32(const int32_t *idx, int64_t batch, int32_t max_active, const 
 /*
  * The backward's sort, run ahead under the forward.  The sort of the slots by
  * feature and its segment starts depend on the indices only, so
- * sft_ft_fwd_f32_prep sorts them into a prepared buffer on a side stream while
- * its forward kernels run (joined before it returns), and
+ * sft_ft_fwd_f32_prep sorts them into a prepared buffer -- on a side stream while
+ * its forward kernels run (joined before it returns), or for a sort too small for
+ * the fork to pay, and outside a stream capture, on the caller's stream ahead of
+ * them -- and
  * sft_ft_bwd_f32_prepared takes that buffer instead of sorting: its critical
  * path is the bias pass and the gathers alone.  Results are those of
  * sft_ft_fwd_f32_ex and sft_ft_bwd_f32, bit for bit.  The buffer must be

@@ -25,7 +25,7 @@ from sft_amd import _native
 
 # ---- SparseLinearFunction (FT/functions.py:12-72) ----
 # The forward also sorts the indices for the backward (the sort needs nothing
-# else), on a side stream beside its gather, into a buffer the autograd
+# else), on a side stream beside its gather or, small ones, ahead of it, into a buffer the autograd
 # Function keeps until its backward: the backward then runs the bias pass and
 # the gathers only.  The reference sorts inside the backward (FT/kernel.py:108-138).
 @torch.library.custom_op("sft::sparse_linear_fwd", mutates_args=(), device_types="cuda")
